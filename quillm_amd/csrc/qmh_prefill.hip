@@ -6,15 +6,16 @@
 //   * activations are quantized per token row exactly as qm_quantize_row_q8 does (src/quant.c);
 //   * a matmul row (r, token p) is the reference's serial chain s = +0; s = s + (float)acc_b *
 //     (dw_b * dx_b) over blocks b in order (src/kernels_scalar.c:12-34). acc_b, the exact int32
-//     dot of one 32-element block, comes from one v_mfma_i32_16x16x32_i8 with a zero
-//     accumulator (16 rows x 16 tokens x one block per instruction); each lane then extends the
-//     float chains of its 4 (row, token) pairs;
+//     dot of one 32-element block, comes from one i8 MFMA with a zero accumulator (32 rows x 32
+//     tokens x one block per v_mfma_i32_32x32x32_i8, or 16 x 16 per v_mfma_i32_16x16x32_i8); the
+//     float chains are extended in block order;
 //   * attention scores, softmax and the weighted V sum keep the decode kernels' per-element
 //     orders (serial over head_dim, the reference softmax, serial over positions).
 //
-// MFMA operand layout (v_mfma_i32_16x16x32_i8, checked on the device): A[i][k] in lane
+// MFMA operand layouts (checked on the device): v_mfma_i32_16x16x32_i8 has A[i][k] in lane
 // i + 16*(k/8), byte k%8; B[k][j] in lane j + 16*(k/8), byte k%8; D[i][j] in lane j + 16*(i/4),
-// element i%4. Any permutation of k applied to both operands leaves the dot unchanged; for
+// element i%4. v_mfma_i32_32x32x32_i8 has A[i][k] in lane i + 32*(k/16), byte k%16, B alike, and
+// D[i][j] in lane j + 32*((i/4)%2), element 4*(i/8) + i%4. Any permutation of k applied to both operands leaves the dot unchanged; for
 // Q4_0 weights each 8-element group is taken as [e0 e2 e4 e6 e1 e3 e5 e7] (the low nibbles of
 // 4 bytes, then the high nibbles), and activations are stored in the same order.
 #include "qmh_device.h"
@@ -26,6 +27,8 @@
 typedef int pf_v4i __attribute__((ext_vector_type(4)));
 typedef float pf_v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 pf_v4h __attribute__((ext_vector_type(4)));
+typedef int pf_v16i __attribute__((ext_vector_type(16)));
+typedef float pf_v16f __attribute__((ext_vector_type(16)));
 
 // ============================================================================ embedding
 
@@ -289,10 +292,6 @@ extern "C" int qmh_launch_pf_quant(const float *x, int ldx, const float *w, floa
 
 // ============================================================================ matmul
 //
-// One wave: NR 16-row tiles x TW 16-token tiles, all blocks in order; 4 waves per workgroup
-// take consecutive 16*NR-row groups of one token group. Operands come straight from memory
-// (weights once per token group, activations from L2), PD blocks ahead of the multiplies.
-
 __device__ __forceinline__ long pf_q4_operand(uint32_t w) {
     // 8 nibbles -> 8 signed int8 (q - 8): low nibbles (e0 e2 e4 e6), then high (e1 e3 e5 e7).
     // Per byte, q + 0x78 stays below 0x100 (no carry into the next byte), and flipping its top
@@ -312,13 +311,12 @@ __device__ __forceinline__ uint32_t pf_slot0(const qmh_pf_args &a, int row, int 
     return (uint32_t)(row / a.tile_r) * a.nb * a.tile_r + row % a.tile_r;
 }
 
-// NM: matrices per wave (2 for the W1 | W3 SwiGLU pair); NR: 16-row tiles per wave (each
-// activation operand feeds NM*NR MFMAs); TW: 16-token tiles per wave
-template <int NM, int NR, int TW>
+// The skinny matmul's operands of one block: NM matrices (2 for the W1 | W3 SwiGLU pair), one 16-row
+// tile, TW 16-token tiles
+template <int NM, int TW>
 struct PfBlock {
-    long A[NM][NR];   // raw weight codes: 8 int8 (Q8_0) or 4 nibble bytes (Q4_0, low word)
-    uint2 sc[NM][NR]; // the fp16 scales of the lane's 4 D rows (k_sk_gemm)
-    uint32_t wh[NM][NR];  // the fp16 scale of the lane's A row (k_pf_gemm)
+    long A[NM];       // raw weight codes: 8 int8 (Q8_0) or 4 nibble bytes (Q4_0, low word)
+    uint32_t wh[NM];  // the fp16 scale of the lane's A row
     long B[TW];
     float dx[TW];
 };
@@ -327,83 +325,30 @@ struct PfBlock {
 // block's uniform base, so the loads take a scalar base and these offsets. Rows past the
 // allocated slots read row 0 instead: each D row depends only on its own A row, and those rows
 // are never stored.
-template <int NM, int NR>
+template <int NM>
 struct PfLane {
-    uint32_t a[NM][NR], s[NM][NR];  // weight codes (bytes), scales (elements) at block 0
-    uint32_t w[NM][NR];             // k_pf_gemm: the scale (element) of the lane's A row at block 0
-    uint32_t x, d;                  // activation codes (bytes), scales (elements) of token tile 0
+    uint32_t a[NM], w[NM];  // weight codes (bytes) and the scale (element) of the lane's A row at block 0
+    uint32_t x, d;          // activation codes (bytes), scales (elements) of token tile 0
 };
 
-// Loads only: no value is used here, so the wait for these loads falls where the block is
-// multiplied, PD blocks later.
-// PM: the scales as k_pf_gemm takes them (one per A row, for the scale MFMA), else the 4 of the
-// lane's D rows.
-template <int WT, int NM, int NR, int TW, bool PM = false>
-__device__ __forceinline__ void pf_load(const qmh_pf_args &a, int b, const PfLane<NM, NR> &ln,
-                                        PfBlock<NM, NR, TW> &o) {
+// Loads only: no value is used here, so the wait for these loads falls where the block is multiplied.
+template <int WT, int NM, int TW>
+__device__ __forceinline__ void pf_load(const qmh_pf_args &a, int b, const PfLane<NM> &ln, PfBlock<NM, TW> &o) {
     constexpr int CB = WT == QMH_Q8 ? 32 : 16;
     const uint8_t *cb = a.codes + (size_t)b * a.tile_r * CB;
     const uint16_t *sb = a.scales + (size_t)b * a.tile_r;
 #pragma unroll
-    for (int m = 0; m < NM; m++)
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            if (WT == QMH_Q8) o.A[m][r] = *(const long *)(cb + ln.a[m][r]);
-            else o.A[m][r] = (long)*(const uint32_t *)(cb + ln.a[m][r]);
-            if (PM) o.wh[m][r] = sb[ln.w[m][r]];
-            else o.sc[m][r] = *(const uint2 *)(sb + ln.s[m][r]);
-        }
+    for (int m = 0; m < NM; m++) {
+        if (WT == QMH_Q8) o.A[m] = *(const long *)(cb + ln.a[m]);
+        else o.A[m] = (long)*(const uint32_t *)(cb + ln.a[m]);
+        o.wh[m] = sb[ln.w[m]];
+    }
     const int8_t *xb = a.xc + (size_t)b * a.PP * 32;
     const float *db = a.xd + (size_t)b * a.PP;
 #pragma unroll
     for (int tt = 0; tt < TW; tt++) {
         o.B[tt] = *(const long *)(xb + ln.x + tt * 512);
         o.dx[tt] = db[ln.d + tt * 16];
-    }
-}
-
-// one block into the chains: s = s + (float)acc * (dw * dx) per (row, token) pair. Two MFMAs per
-// (row tile, token tile): the block's exact int32 dots, and the scale products dw * dx as the outer
-// product of the row tile's 16 fp16 scales and the token tile's 16 (k = 0 of an f16 MFMA; every
-// other k is 0 * 0). The product of two fp16 values is exact in fp32, so the MFMA returns the
-// reference's dw * dx bit for bit (but +0 for -0: the chain starts at +0 and never holds -0, so
-// s + (+0) == s + (-0) and the term's zero sign changes nothing); the VALU keeps the conversion,
-// the multiply and the add, in the reference's order. k0 is 0xffff in the lanes of k = 0..3
-// (lane / 16 == 0), else 0.
-// The MFMAs of the next (row tile, token tile) pair go out, into their own registers, before the
-// terms of the current one, so the multiplies run under the float work instead of each waiting for
-// the previous results to be consumed. Every accumulator's chain stays in block order.
-template <int WT, int NM, int NR, int TW>
-__device__ __forceinline__ void pf_mul(const PfBlock<NM, NR, TW> &cur, float (&s)[NM][NR][TW][4], uint32_t k0) {
-    constexpr int Q = NM * NR, U = Q * TW;  // pair u: row tile (m, r) = (q / NR, q % NR), q = u / TW; tt = u % TW
-    pf_v4h Bs[TW];                          // token tile tt's scales at k = 0
-#pragma unroll
-    for (int tt = 0; tt < TW; tt++) {
-        const uint32_t h = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)cur.dx[tt]) & k0;  // exact: dx is fp16
-        Bs[tt] = __builtin_bit_cast(pf_v4h, make_uint2(h, 0u));
-    }
-    long Am[Q];
-    pf_v4h As[Q];  // row tile q's scales at k = 0
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-        Am[q] = WT == QMH_Q8 ? cur.A[q / NR][q % NR] : pf_q4_operand((uint32_t)cur.A[q / NR][q % NR]);
-        As[q] = __builtin_bit_cast(pf_v4h, make_uint2(cur.wh[q / NR][q % NR] & k0, 0u));
-    }
-    pf_v4i acc[2];
-    pf_v4f pw[2];
-    auto issue = [&](int u, pf_v4i &d, pf_v4f &pd) {
-        const pf_v4i z = {0, 0, 0, 0};
-        const pf_v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
-        d = __builtin_amdgcn_mfma_i32_16x16x32_i8(Am[u / TW], cur.B[u % TW], z, 0, 0, 0);
-        pd = __builtin_amdgcn_mfma_f32_16x16x16f16(As[u / TW], Bs[u % TW], zf, 0, 0, 0);
-    };
-    issue(0, acc[0], pw[0]);
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        if (u + 1 < U) issue(u + 1, acc[(u + 1) & 1], pw[(u + 1) & 1]);
-        const int q = u / TW, m = q / NR, r = q % NR, tt = u % TW;
-#pragma unroll
-        for (int e = 0; e < 4; e++) s[m][r][tt][e] = s[m][r][tt][e] + (float)acc[u & 1][e] * pw[u & 1][e];
     }
 }
 
@@ -432,113 +377,326 @@ __device__ __forceinline__ void pf_store(const qmh_pf_args &a, int row, int p, f
     }
 }
 
-template <int WT, int NM, int NR, int TW, int PD>
-__global__ __launch_bounds__(QMH_WG) void k_pf_gemm(qmh_pf_args a) {
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, kq = l >> 4;
-    const int r0 = (blockIdx.y * (QMH_WG / 64) + wave) * 16 * NR;  // the wave's 16*NR rows
-    const int t0 = blockIdx.x * 16 * TW;                           // the wave's first token
-    if (r0 >= a.rows) return;
+// ---- tiled matmul (more than QMH_PF_SKINNY_P tokens)
+//
+// A workgroup owns RT 32-row tiles x TT 32-token tiles, one (row tile, token tile) pair per wave, and
+// takes all blocks in order. IL (W1 | W3): the first RT/2 row tiles are W1 rows, the others the same
+// rows of W3, whose values pass to the W1 waves through LDS at the end.
+//
+// What bounds it. Per 1024 outputs (32 x 32) and block a wave issues 48 VALU instructions (convert,
+// multiply, add: the reference's three roundings) and two MFMAs of 32 cycles. On this device a SIMD takes
+// a VALU instruction every 2 cycles from two or more waves (every 4 from one), and an MFMA's cycles
+// largely add to the VALU's: about 163 cycles per pair of tile and block, and the clock falls to
+// ~1.9 GHz under it. So the shape that needs the fewest cycles wins, not the one with the most work per
+// load: v_mfma_i32_32x32x32_i8 gives 1024 dots in 32 cycles where 16x16x32 takes 64, and likewise the
+// f16 32x32x8 for the scale products. Timed at 512 tokens (us, 16x16 tiles in registers -> this):
+// 12288x4096 150 -> 99, 4096x4096 57 -> 41, W1|W3 2x11008x4096 230 -> 186, 4096x11008 143 -> 95.
+// Tried and slower: the int8 accumulator started at the bits of 1.5*2^23 with a second scale product
+// -1.5*2^23*dw*dx, for two VALU instructions per term (an f32 MFMA runs on the VALU's own units, and
+// the third MFMA costs what the conversion saved); 32x32 tiles with operands straight from
+// memory (105, 45, 198, 99: the loads bound it); two token tiles per wave (one wave per SIMD).
+//
+// Operands pass through LDS in stages of PG_KB blocks, two buffers: a thread's pieces of stage i + 2
+// (+ DEEP) are loaded to registers during stage i and written when stage i has been read. The loads'
+// offsets are fixed per thread (buffer loads, the block in the scalar offset; the resource's size
+// zeroes what lies past the matrix), and the barrier waits for LDS only, so loads stay in flight
+// across it. Q4_0 codes are written as 16*(q - 8) (two operations per four codes; a chain of 16 x the
+// terms is 16 x the reference's chain exactly, so one multiply by 1/16 ends it: no term is below
+// 2^-48 or above 2^52). In LDS each half block of every row (or token) is contiguous over the rows,
+// which has no bank conflicts; the four fp16 scales of a row sit side by side, and the scale product of
+// block j takes all four as k = 0..3 of A against B with only entry j (others 0).
+//
+// Inside a block: convert and multiply by the scale products, issue the next block's integer MFMA
+// (its accumulators are free), add to the chains, issue the next block's scale MFMA.
+//
+// Infinite or NaN scales: 0 * inf in the scale MFMA makes a NaN where the reference might not, and
+// leaves a NaN in every chain it touches, so rows that end as NaN are computed again from memory
+// (pg_row). Finite scales never give a NaN or an infinity.
+#define PG_KB 4
+#define PG_FENCE() __builtin_amdgcn_sched_barrier(0)  // keeps the order above
+
+// every LDS access done, then the barrier: the vector memory loads in flight are not waited for
+__device__ __forceinline__ void pg_lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int RT, int TT>
+struct PgLds {
+    static constexpr int A = PG_KB * RT * 1024, B = PG_KB * TT * 1024, W = RT * 32 * 8, D = TT * 32 * 8;
+    static constexpr int STG = A + B + W + D;
+};
+
+// one row's chain from memory, block by block as the reference (a row or token with an infinite or NaN
+// scale, see k_pf_gemm)
+template <int WT>
+__device__ float pg_row(const qmh_pf_args &a, uint32_t slot, int p) {
     constexpr int CB = WT == QMH_Q8 ? 32 : 16;
-    PfLane<NM, NR> ln;
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-        const int row = r0 + 16 * r + (l & 15);  // the lane's A row
-#pragma unroll
-        for (int m = 0; m < NM; m++) {
-            ln.a[m][r] = pf_slot0(a, row < a.rows_alloc ? row : 0, m) * CB + (WT == QMH_Q8 ? 8 : 4) * kq;
-            ln.w[m][r] = pf_slot0(a, row < a.rows_alloc ? row : 0, m);
+    float s = 0.0f;
+#pragma unroll 1
+    for (int b = 0; b < a.nb; b++) {
+        const uint8_t *c = a.codes + ((size_t)slot + (size_t)b * a.tile_r) * CB;
+        const int8_t *x = a.xc + ((size_t)b * a.PP + p) * 32;
+        int acc = 0;
+#pragma unroll 1
+        for (int g = 0; g < 8; g++) {  // 4 image bytes; Q4_0: group 8 * (g / 2), low nibbles then high
+            const uint32_t xw = *(const uint32_t *)(x + 4 * g);
+            uint32_t w;
+            if (WT == QMH_Q8) w = *(const uint32_t *)(c + 4 * g);
+            else w = (uint32_t)(pf_q4_operand(*(const uint32_t *)(c + 4 * (g >> 1))) >> (32 * (g & 1)));
+            acc = __builtin_amdgcn_sdot4((int)w, (int)xw, acc, false);
         }
+        const float dw = qmh_h2f(a.scales[(size_t)slot + (size_t)b * a.tile_r]);
+        s = s + (float)acc * (dw * a.xd[(size_t)b * a.PP + p]);
     }
-    ln.x = (uint32_t)(t0 + (l & 15)) * 32 + 8 * kq;
-    ln.d = (uint32_t)(t0 + (l & 15));
-    const uint32_t k0 = kq == 0 ? 0xffffu : 0u;
-    float s[NM][NR][TW][4];
+    return s;
+}
+
+template <int WT, bool IL, int RT, int TT, int DEEP>
+__global__ __launch_bounds__(64 * RT * TT, 4) void k_pf_gemm(qmh_pf_args a) {
+    constexpr int KB = PG_KB, CB = WT == QMH_Q8 ? 32 : 16, AH = CB / 16, WG = 64 * RT * TT;
+    constexpr int NR = RT * 32, NTK = TT * 32, RS = WG / NR, TS = WG / NTK;
+    constexpr int NA = KB / RS, NB = 2 * KB / TS, ND = (KB + TS - 1) / TS;
+    using L = PgLds<RT, TT>;
+    __shared__ __align__(16) uint8_t lds[2 * L::STG];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, hi = l >> 5, lr = l & 31;
+    // workgroups go round robin over the 8 XCDs: the token groups of a row group share one XCD's L2
+    // (W1 | W3 at 512 tokens 217 -> 208 us)
+    const int gx = gridDim.x, gy = gridDim.y, lin = blockIdx.y * gx + blockIdx.x;
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (lin < gy / 8 * 8 * gx) {
+        by = (lin >> 3) / gx * 8 + (lin & 7);
+        bx = (lin >> 3) % gx;
+    }
+    const int rg0 = by * (IL ? NR / 2 : NR), t0 = bx * NTK, nb = a.nb;
+    const int row = tid % NR, j0 = tid / NR;    // A: row of the tile, blocks j0 + k*RS
+    const int tok = tid % NTK, q0 = tid / NTK;  // B: token, (half, block) q0 + k*TS
+    // offsets from the workgroup's first slot; rows past the allocated ones read its first row
+    const uint32_t slot_w = pf_slot0(a, rg0, 0);
+    auto slot_of = [&](int r) {
+        const int rr = rg0 + (IL ? r % (NR / 2) : r);
+        return pf_slot0(a, rr < a.rows_alloc ? rr : rg0, IL ? r / (NR / 2) : 0);
+    };
+    const uint32_t slot_r = slot_of(row) - slot_w;
+    const size_t nslots = (size_t)(IL ? a.rows_alloc / (a.tile_r / 2) * a.tile_r : a.rows_alloc) * nb - slot_w;
+    auto rsrc = [](const void *q, size_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)q, (short)0, (int)(bytes < 0xffffffffu ? bytes : 0xffffffffu), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rca = rsrc(a.codes + (size_t)slot_w * CB, nslots * CB), rcw = rsrc(a.scales + slot_w, nslots * 2);
+    const __amdgpu_buffer_rsrc_t rcb = rsrc(a.xc + (size_t)t0 * 32, ((size_t)nb * a.PP - t0) * 32);
+    const __amdgpu_buffer_rsrc_t rcd = rsrc(a.xd + t0, ((size_t)nb * a.PP - t0) * 4);
+    const uint32_t ast = (uint32_t)a.tile_r * CB, bst = (uint32_t)a.PP * 32;
+    const uint32_t va = slot_r * CB + j0 * ast, vw = (slot_r + j0 * a.tile_r) * 2;
+    const uint32_t vb = tok * 32 + (q0 & 1) * 16 + (q0 >> 1) * bst, vd = (uint32_t)(tok + q0 * a.PP) * 4;
+    pf_v4u ra_[1 + DEEP][NA][AH], rb_[1 + DEEP][NB];
+    uint32_t rw_[1 + DEEP][NA], rd_[1 + DEEP][ND];
+    // stage of blocks b0.. into register set q, and from there to the LDS buffer at base
+    auto gload = [&](int b0, int q) {
 #pragma unroll
-    for (int m = 0; m < NM; m++)
+        for (int k = 0; k < NA; k++) {
 #pragma unroll
-        for (int r = 0; r < NR; r++)
-#pragma unroll
-            for (int tt = 0; tt < TW; tt++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) s[m][r][tt][e] = 0.0f;
-    // PD blocks in flight ahead of the one multiplied: a ring of PD + 1 operand sets indexed
-    // statically (the group loop is unrolled PD + 1 times), so no operand is copied and each
-    // wait is for loads issued PD blocks earlier. Invariant at the top of a group starting at
-    // block b0: ring[j] holds block b0 + j, j < PD.
-    PfBlock<NM, NR, TW> ring[PD + 1];
-#pragma unroll
-    for (int j = 0; j < PD; j++) pf_load<WT, NM, NR, TW, true>(a, j < a.nb ? j : a.nb - 1, ln, ring[j]);
-    int b0 = 0;
-    for (; b0 + PD < a.nb; b0 += PD + 1) {
-#pragma unroll
-        for (int j = 0; j <= PD; j++) {
-            const int bn = b0 + j + PD;
-            pf_load<WT, NM, NR, TW, true>(a, bn < a.nb ? bn : a.nb - 1, ln, ring[(j + PD) % (PD + 1)]);
-            pf_mul<WT, NM, NR, TW>(ring[j], s, k0);
+            for (int h = 0; h < AH; h++)
+                ra_[q][k][h] = __builtin_amdgcn_raw_buffer_load_b128(rca, va + 16 * h, (b0 + k * RS) * ast, 0);
+            rw_[q][k] = __builtin_amdgcn_raw_buffer_load_b16(rcw, vw, (b0 + k * RS) * a.tile_r * 2, 0);
         }
-    }
 #pragma unroll
-    for (int j = 0; j < PD; j++)
-        if (b0 + j < a.nb) pf_mul<WT, NM, NR, TW>(ring[j], s, k0);
-    // epilogues: lane l holds rows r0 + 16*r + 4*kq + e (e < 4) of tokens t0 + 16*tt + l%16
-    if (NR == 2 && a.epi == QMH_PF_SWIGLU && a.qxc) {  // uniform
-        // W2's input as its Q8_0 image: the wave's 32 rows (r0 % 32 == 0) are block r0/32 of each of
-        // its tokens; lanes l, l^16, l^32, l^48 hold a token's 32 values (8 each: elements
-        // 16*r + 4*kq + e). The same steps as k_pf_quant's block (src/quant.c:27-52): amax, the fp16
-        // scale, the codes; rows past `rows` are 0 there and here.
-        const int b = r0 >> 5;
+        for (int k = 0; k < NB; k++) rb_[q][k] = __builtin_amdgcn_raw_buffer_load_b128(rcb, vb, (b0 + k * (TS / 2)) * bst, 0);
 #pragma unroll
-        for (int tt = 0; tt < TW; tt++) {
-            const int p = t0 + 16 * tt + (l & 15);
-            float v[NR][4], m = 0.0f;
+        for (int k = 0; k < ND; k++)
+            if (TS <= KB || wave * 64 / NTK < KB) rd_[q][k] = __builtin_amdgcn_raw_buffer_load_b32(rcd, vd, (b0 + k * TS) * a.PP * 4, 0);
+    };
+    auto swrite = [&](uint32_t base, int q) {
 #pragma unroll
-            for (int r = 0; r < NR; r++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int row = r0 + 16 * r + 4 * kq + e;
-                    const float y = s[0][r][tt][e], up = s[NM - 1][r][tt][e];
-                    v[r][e] = row < a.rows ? y / (1.0f + qmh_expf(-y)) * up : 0.0f;  // silu(g)*u (src/ops.c:128-133)
-                    const float av = fabsf(v[r][e]);
-                    m = av > m ? av : m;
-                }
-            float o = __shfl_xor(m, 16);
-            m = o > m ? o : m;
-            o = __shfl_xor(m, 32);
-            m = o > m ? o : m;
-            const float dd = qmh_h2f(qmh_f2h(qmh_div127(m)));
-            const float rinv = qmh_rcp(dd);
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                int q[4];
-                qmh_q8_codes4(v[r], dd, rinv, q);
-                const uint32_t b0 = (uint32_t)q[0] & 0xffu, b1 = (uint32_t)q[1] & 0xffu, b2 = (uint32_t)q[2] & 0xffu,
-                               b3 = (uint32_t)q[3] & 0xffu;
-                // bytes 16*r + 4*kq .. +3 of the block; the Q4_0 order (8g+e at 8g + {0,4,1,5,2,6,3,7}[e])
-                // by a half-word swap with lane l^16, as in k_pf_quant
-                const uint32_t pk = b0 | (b2 << 8) | (b1 << 16) | (b3 << 24);
-                const uint32_t pp = (uint32_t)__shfl_xor((int)pk, 16);
-                const uint32_t w = !a.qperm8 ? (b0 | (b1 << 8) | (b2 << 16) | (b3 << 24))
-                                   : (kq & 1) == 0 ? ((pk & 0xffffu) | (pp << 16)) : ((pp >> 16) | (pk & 0xffff0000u));
-                if (p < a.P) *(uint32_t *)(a.qxc + ((size_t)b * a.PP + p) * 32 + 16 * r + 4 * kq) = w;
+        for (int k = 0; k < NA; k++) {
+            pf_v4u lo = ra_[q][k][0], hh = ra_[q][k][AH - 1];
+            if (WT == QMH_Q4) {
+                const pf_v4u v = lo;
+                lo[0] = ((v[0] << 4) & 0xf0f0f0f0u) ^ 0x80808080u, lo[1] = (v[0] & 0xf0f0f0f0u) ^ 0x80808080u;
+                lo[2] = ((v[1] << 4) & 0xf0f0f0f0u) ^ 0x80808080u, lo[3] = (v[1] & 0xf0f0f0f0u) ^ 0x80808080u;
+                hh[0] = ((v[2] << 4) & 0xf0f0f0f0u) ^ 0x80808080u, hh[1] = (v[2] & 0xf0f0f0f0u) ^ 0x80808080u;
+                hh[2] = ((v[3] << 4) & 0xf0f0f0f0u) ^ 0x80808080u, hh[3] = (v[3] & 0xf0f0f0f0u) ^ 0x80808080u;
             }
-            if (p < a.P && kq == 0) a.qxd[(size_t)b * a.PP + p] = dd;
+            uint8_t *o = lds + base + (j0 + k * RS) * (NR * 32) + row * 16;
+            *(pf_v4u *)o = lo;
+            *(pf_v4u *)(o + NR * 16) = hh;
+            *(uint16_t *)(lds + base + L::A + L::B + row * 8 + 2 * (j0 + k * RS)) = (uint16_t)rw_[q][k];
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++)
+            *(pf_v4u *)(lds + base + L::A + (q0 + k * TS) * (NTK * 16) + tok * 16) = rb_[q][k];
+#pragma unroll
+        for (int k = 0; k < ND; k++)
+            if (TS <= KB || wave * 64 / NTK < KB)
+                *(_Float16 *)(lds + base + L::A + L::B + L::W + tok * 8 + 2 * (q0 + k * TS)) = (_Float16)__uint_as_float(rd_[q][k]);
+    };
+    // the wave's operands: codes by block parity, scales by stage parity
+    const int wr = wave / TT, wt = wave % TT;
+    const uint32_t oa = hi * (NR * 16) + (uint32_t)(wr * 32 + lr) * 16, ob = L::A + hi * (NTK * 16) + (uint32_t)(wt * 32 + lr) * 16;
+    const uint32_t ow = L::A + L::B + (uint32_t)(wr * 32 + lr) * 8, od = L::A + L::B + L::W + (uint32_t)(wt * 32 + lr) * 8;
+    const uint32_t mlo = hi ? 0 : 0xffffu, mhi = hi ? 0 : 0xffff0000u;
+    pf_v4i A[2], B[2];
+    uint2 w[2], d[2];
+    auto rd = [&](uint32_t base, int j, int k) {
+        A[k] = *(const pf_v4i *)(lds + base + oa + j * (NR * 32));
+        B[k] = *(const pf_v4i *)(lds + base + ob + j * (NTK * 32));
+    };
+    auto rs = [&](uint32_t base, int k) {
+        w[k] = *(const uint2 *)(lds + base + ow);
+        d[k] = *(const uint2 *)(lds + base + od);
+    };
+    float s[16];
+    pf_v16i acc, zi;
+    pf_v16f pw, zf;
+#pragma unroll
+    for (int e = 0; e < 16; e++) s[e] = 0.0f, zi[e] = 0, zf[e] = 0.0f;
+    auto isp = [&](int k, int j) {
+        const uint2 m = j == 0 ? make_uint2(d[k].x & mlo, 0u) : j == 1 ? make_uint2(d[k].x & mhi, 0u)
+                        : j == 2 ? make_uint2(0u, d[k].y & mlo) : make_uint2(0u, d[k].y & mhi);
+        pw = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(pf_v4h, w[k]), __builtin_bit_cast(pf_v4h, m), zf, 0, 0, 0);
+    };
+    auto isi = [&](int k) { acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[k], B[k], zi, 0, 0, 0); };
+    // the block whose MFMAs are in flight into the chains; the next block's MFMAs from operand set k,
+    // entry j of scale set sk
+    auto mul = [&](int k, int sk, int j) {
+        PG_FENCE();
+        float f[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) f[e] = (float)acc[e];
+        PG_FENCE();
+#pragma unroll
+        for (int e = 0; e < 16; e++) f[e] = f[e] * pw[e];
+        PG_FENCE();
+        isi(k);
+        PG_FENCE();
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = s[e] + f[e];
+        PG_FENCE();
+        isp(sk, j);
+        PG_FENCE();
+    };
+    const int nst = (nb + KB - 1) / KB;
+    gload(0, 0);
+    if (DEEP) gload(KB, DEEP);
+    swrite(0, 0);
+    if (!DEEP) gload(KB, 0);
+    else gload(2 * KB, 0);
+    pg_lds_barrier();
+    swrite(L::STG, DEEP);
+    gload((2 + DEEP) * KB, DEEP);
+    rd(0, 0, 0);
+    rd(0, 1, 1);
+    rs(0, 0);
+    isi(0), isp(0, 0);
+    for (int i0 = 0; i0 < nst; i0 += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int b0 = (i0 + h) * KB;
+            const uint32_t base = h * L::STG, oth = L::STG - base;
+#pragma unroll
+            for (int j = 0; j < KB; j++) {
+                if (j == KB - 2) {
+                    pg_lds_barrier();  // this stage's operands are read, the next stage is written
+                    rd(oth, 0, j & 1);
+                    rs(oth, h ^ 1);
+                    swrite(base, DEEP ? h : 0);
+                    gload(b0 + (3 + DEEP) * KB, DEEP ? h : 0);
+                } else {
+                    rd(j < KB - 2 ? base : oth, (j + 2) % KB, j & 1);
+                }
+                if (b0 + j < nb) mul((j & 1) ^ 1, j == KB - 1 ? h ^ 1 : h, (j + 1) % KB);
+            }
+        }
+    }
+    if (WT == QMH_Q4)
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = s[e] * 0.0625f;
+    const int p = t0 + 32 * wt + lr, wrow = rg0 + 32 * (IL ? wr % (RT / 2) : wr);
+    // a NaN here means an infinite or NaN scale: that row's chain again, from memory
+    uint32_t nan = 0;
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+        nan |= (s[e] != s[e] && p < a.P && wrow + 8 * (e >> 2) + 4 * hi + (e & 3) < a.rows) ? 1u << e : 0u;
+    if (__any(nan != 0)) {
+#pragma unroll 1
+        for (int e = 0; e < 16; e++) {
+            if (!((nan >> e) & 1)) continue;
+            const float v = pg_row<WT>(a, pf_slot0(a, wrow + 8 * (e >> 2) + 4 * hi + (e & 3), IL ? wr / (RT / 2) : 0), p);
+#pragma unroll
+            for (int k = 0; k < 16; k++) s[k] = k == e ? v : s[k];
+        }
+    }
+    if (!IL) {
+        if (p >= a.P) return;
+        // 4 consecutive rows per lane: 16-byte accesses where they are whole and aligned
+        if ((a.epi == QMH_PF_STORE || a.epi == QMH_PF_ADD) && a.ld0 % 4 == 0 && ((uintptr_t)a.out0 & 15) == 0 &&
+            rg0 + NR <= a.rows) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                pf_v4f *o = (pf_v4f *)(a.out0 + (size_t)p * a.ld0 + wrow + 8 * g + 4 * hi);
+                pf_v4f y = {s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
+                if (a.epi == QMH_PF_ADD) {  // x += W x' (src/model.c:179,186)
+                    const pf_v4f x = *o;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) y[e] = x[e] + y[e];
+                }
+                *o = y;
+            }
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int r = wrow + 8 * (e >> 2) + 4 * hi + (e & 3);
+            if (r < a.rows) pf_store(a, r, p, s[e], 0.0f, s[e ^ 1]);
         }
         return;
     }
+    // W3's values to the waves of W1
+    __syncthreads();
+    constexpr int HW = RT / 2 * TT;  // waves of W1
+    float *x = (float *)lds + (wave % HW) * 1024 + l;
+    static_assert(2 * L::STG >= HW * 4096, "the exchange fits the stages");
+    if (wave >= HW)
 #pragma unroll
-    for (int r = 0; r < NR; r++)
+        for (int e = 0; e < 16; e++) x[e * 64] = s[e];
+    __syncthreads();
+    if (wave >= HW) return;
+    float up[16];
 #pragma unroll
-        for (int tt = 0; tt < TW; tt++) {
-            const int p = t0 + 16 * tt + (l & 15);
-            if (p >= a.P) continue;
+    for (int e = 0; e < 16; e++) up[e] = x[e * 64];
+    if (!a.qxc) {
+        if (p >= a.P) return;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = r0 + 16 * r + 4 * kq + e;
-                if (row >= a.rows) continue;
-                // rows 2i, 2i+1 share the lane (RoPE partner)
-                pf_store(a, row, p, s[0][r][tt][e], s[NM - 1][r][tt][e], s[0][r][tt][e ^ 1]);
-            }
+        for (int e = 0; e < 16; e++) {
+            const int r = wrow + 8 * (e >> 2) + 4 * hi + (e & 3);
+            if (r < a.rows) pf_store(a, r, p, s[e], up[e], 0.0f);
         }
+        return;
+    }
+    // W2's input as its Q8_0 image: the wave's 32 rows are one block of each of its tokens, 16 values in
+    // lane l and 16 in l ^ 32. The same steps as k_pf_quant's block (src/quant.c:27-52): amax, the fp16
+    // scale, the codes (Q4_0 order: 8g + e at 8g + {0,4,1,5,2,6,3,7}[e], by a half-word swap with
+    // lane l ^ 32); rows past `rows` are 0 there and here.
+    float v[16], m = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const float y = s[e];
+        v[e] = wrow + 8 * (e >> 2) + 4 * hi + (e & 3) < a.rows ? y / (1.0f + qmh_expf(-y)) * up[e] : 0.0f;  // src/ops.c:128-133
+        const float av = fabsf(v[e]);
+        m = av > m ? av : m;
+    }
+    const float o = __shfl_xor(m, 32);
+    m = o > m ? o : m;
+    const float dd = qmh_h2f(qmh_f2h(qmh_div127(m))), rinv = qmh_rcp(dd);
+    const int b = wrow >> 5;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        int q[4];
+        qmh_q8_codes4(v + 4 * g, dd, rinv, q);
+        const uint32_t c0 = (uint32_t)q[0] & 0xffu, c1 = (uint32_t)q[1] & 0xffu, c2 = (uint32_t)q[2] & 0xffu, c3 = (uint32_t)q[3] & 0xffu;
+        const uint32_t pk = c0 | (c2 << 8) | (c1 << 16) | (c3 << 24);
+        const uint32_t pp = (uint32_t)__shfl_xor((int)pk, 32);
+        const uint32_t wv = !a.qperm8 ? (c0 | (c1 << 8) | (c2 << 16) | (c3 << 24))
+                            : hi == 0 ? ((pk & 0xffffu) | (pp << 16)) : ((pp >> 16) | (pk & 0xffff0000u));
+        if (p < a.P) *(uint32_t *)(a.qxc + ((size_t)b * a.PP + p) * 32 + 8 * g + 4 * hi) = wv;
+    }
+    if (p < a.P && hi == 0) a.qxd[(size_t)b * a.PP + p] = dd;
 }
 
 // Skinny matmul for decode-sized batches (P <= 16*TT tokens, TT <= 4): one workgroup per 16-row group
@@ -566,13 +724,13 @@ __global__ __launch_bounds__(SK_WG) void k_sk_gemm(qmh_pf_args a) {
     const int r0 = blockIdx.x * 16, P = a.P, nb = a.nb;
     const int rblk = sk_round(nb, NM, P);
     constexpr int CB = WT == QMH_Q8 ? 32 : 16;
-    PfLane<NM, 1> ln;
+    PfLane<NM> ln;
     {
         const int row = r0 + tok;  // the lane's A row
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            ln.a[m][0] = pf_slot0(a, row < a.rows_alloc ? row : 0, m) * CB + (WT == QMH_Q8 ? 8 : 4) * kq;
-            ln.w[m][0] = pf_slot0(a, row < a.rows_alloc ? row : 0, m);
+            ln.a[m] = pf_slot0(a, row < a.rows_alloc ? row : 0, m) * CB + (WT == QMH_Q8 ? 8 : 4) * kq;
+            ln.w[m] = pf_slot0(a, row < a.rows_alloc ? row : 0, m);
         }
     }
     const uint32_t kmask = kq == 0 ? 0xffffu : 0u;  // lanes of k = 0..3
@@ -586,11 +744,11 @@ __global__ __launch_bounds__(SK_WG) void k_sk_gemm(qmh_pf_args a) {
     for (int base = 0; base < nb; base += rblk) {
         const int nr = min(rblk, nb - base);
         for (int k0 = 0; 8 * k0 + wave < nr; k0 += PD) {  // uniform per wave
-            PfBlock<NM, 1, TT> blk[PD];
+            PfBlock<NM, TT> blk[PD];
 #pragma unroll
             for (int j = 0; j < PD; j++) {
                 const int jb = 8 * (k0 + j) + wave;
-                pf_load<WT, NM, 1, TT, true>(a, base + (jb < nr ? jb : nr - 1), ln, blk[j]);
+                pf_load<WT, NM, TT>(a, base + (jb < nr ? jb : nr - 1), ln, blk[j]);
             }
 #pragma unroll
             for (int j = 0; j < PD; j++) {
@@ -598,8 +756,8 @@ __global__ __launch_bounds__(SK_WG) void k_sk_gemm(qmh_pf_args a) {
                 if (jb < nr) {  // uniform per wave
                     // every MFMA of the block first, each into its own registers, then the terms:
                     // the multiplies overlap instead of each waiting for the previous results. The
-                    // scale products dw * dx come from an f16 MFMA with the scales at k = 0, as in
-                    // k_pf_gemm (exact: a product of two fp16 values)
+                    // scale products dw * dx come from an f16 MFMA with the scales at k = 0 (exact: a
+                    // product of two fp16 values), as in k_pf_gemm
                     pf_v4i acc[NM][TT];
                     pf_v4f pw[NM][TT];
                     pf_v4h Bs[TT];
@@ -610,8 +768,8 @@ __global__ __launch_bounds__(SK_WG) void k_sk_gemm(qmh_pf_args a) {
                     }
 #pragma unroll
                     for (int m = 0; m < NM; m++) {
-                        const long Am = WT == QMH_Q8 ? blk[j].A[m][0] : pf_q4_operand((uint32_t)blk[j].A[m][0]);
-                        const pf_v4h As = __builtin_bit_cast(pf_v4h, make_uint2(blk[j].wh[m][0] & kmask, 0u));
+                        const long Am = WT == QMH_Q8 ? blk[j].A[m] : pf_q4_operand((uint32_t)blk[j].A[m]);
+                        const pf_v4h As = __builtin_bit_cast(pf_v4h, make_uint2(blk[j].wh[m] & kmask, 0u));
 #pragma unroll
                         for (int tt = 0; tt < TT; tt++) {
                             const pf_v4i z = {0, 0, 0, 0};
@@ -897,20 +1055,12 @@ __global__ __launch_bounds__(BMV_NT, 4) void k_bmv(qmh_pf_args a) {  // 4 waves 
         }
 }
 
-// Wave shape of the matmuls (timed on MI355X at P = 512 over the 7B shapes): 2 row tiles x 4
-// token tiles per wave, 2 blocks loaded ahead. Fewer tiles per wave issue more loads per MFMA;
-// more leave too few waves to cover the latency at P = 512. W1 | W3 loads 1 block ahead: that
-// holds it to 166 VGPRs, three waves per SIMD, so its 2752 wave tiles at P = 512 (7B shapes) run
-// in one round of 3072 slots instead of 1.34 rounds of 2048 (20.45 -> 20.02 ms per 512-token
-// prefill); the other matrices lose at depth 1 (23.5 ms with every one there).
-enum { PF_NR = 2, PF_TW = 4, PF_PD = 2, PF_PD13 = 1 };
-
 extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
     if (a->PP % 128 || a->P > a->PP || a->P < 1 || a->nb < 1) return (int)hipErrorInvalidValue;
     if ((a->epi == QMH_PF_SWIGLU) != (a->il != 0)) return (int)hipErrorInvalidValue;
     if (a->dtype != QMH_Q4 && a->dtype != QMH_Q8) return (int)hipErrorInvalidValue;
     // the image output exists only in the tiled matmul's SwiGLU epilogue (more than QMH_PF_SKINNY_P tokens)
-    if (a->qxc && (a->epi != QMH_PF_SWIGLU || !a->qxd || a->P <= QMH_PF_SKINNY_P || PF_NR != 2)) return (int)hipErrorInvalidValue;
+    if (a->qxc && (a->epi != QMH_PF_SWIGLU || !a->qxd || a->P <= QMH_PF_SKINNY_P)) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
     if (a->xf && (a->nxf < 1 || a->nxf > 32 * a->nb || a->ldxf < a->nxf)) return (int)hipErrorInvalidValue;
     // the multi-token matvec when one tile's terms fit its LDS with the records. It quantizes a plain
@@ -985,16 +1135,25 @@ extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
 #undef SK_LAUNCH
         return (int)hipGetLastError();
     }
-    // token groups past P are not launched; 16 * PF_TW divides PP, so every B load stays in the
-    // PP-token activation buffer
-    const dim3 g((a->P + 16 * PF_TW - 1) / (16 * PF_TW), (a->rows + 64 * PF_NR - 1) / (64 * PF_NR));
-    if (a->il) {
-        if (a->dtype == QMH_Q4) hipLaunchKernelGGL((k_pf_gemm<QMH_Q4, 2, PF_NR, PF_TW, PF_PD13>), g, dim3(QMH_WG), 0, s, *a);
-        else hipLaunchKernelGGL((k_pf_gemm<QMH_Q8, 2, PF_NR, PF_TW, PF_PD13>), g, dim3(QMH_WG), 0, s, *a);
-    } else {
-        if (a->dtype == QMH_Q4) hipLaunchKernelGGL((k_pf_gemm<QMH_Q4, 1, PF_NR, PF_TW, PF_PD>), g, dim3(QMH_WG), 0, s, *a);
-        else hipLaunchKernelGGL((k_pf_gemm<QMH_Q8, 1, PF_NR, PF_TW, PF_PD>), g, dim3(QMH_WG), 0, s, *a);
-    }
+    // the tiled matmul. Token groups past P are not launched, and 64 divides PP, so every read of the
+    // activations stays in the PP-token image. 4 x 2 tiles per workgroup, two waves per SIMD of a CU;
+    // 2 x 2 where 4 x 2 would leave half of the CUs idle or more (timed, us, 4 x 2 -> 2 x 2: 4096x11008 at
+    // 96 tokens, 64 workgroups, 82 -> 66; 2048x5632 at 512, 128, 47 -> 39; 4096x4096 at 300, 160,
+    // 36.7 -> 37.8) and for W1 | W3, whose 64-slot tiles it reads whole (4096 columns: 197 -> 186; 2048:
+    // 59 -> 60), both with the loads two stages ahead.
+    const int tg = (a->P + 63) / 64, g4 = tg * ((a->rows + 127) / 128);
+#define PG_LAUNCH(IL_, RT_, DEEP_, ROWS_)                                                                                \
+    do {                                                                                                                 \
+        const dim3 g(tg, (a->rows + (ROWS_)-1) / (ROWS_));                                                               \
+        if (a->dtype == QMH_Q4)                                                                                          \
+            hipLaunchKernelGGL((k_pf_gemm<QMH_Q4, IL_, RT_, 2, DEEP_>), g, dim3(128 * RT_), 0, s, *a);                \
+        else                                                                                                             \
+            hipLaunchKernelGGL((k_pf_gemm<QMH_Q8, IL_, RT_, 2, DEEP_>), g, dim3(128 * RT_), 0, s, *a);                \
+    } while (0)
+    if (a->il) PG_LAUNCH(true, 2, 1, 32);
+    else if (g4 <= 128) PG_LAUNCH(false, 2, 1, 64);
+    else PG_LAUNCH(false, 4, 0, 128);
+#undef PG_LAUNCH
     return (int)hipGetLastError();
 }
 
