@@ -99,6 +99,26 @@ __device__ __forceinline__ float qmh_expf_t(float x, const uint64_t *tab) {
     return (float)y;
 }
 __device__ __forceinline__ float qmh_expf(float x) { return qmh_expf_t(x, qmh_exp2_tab); }
+// qmh_expf_t(x, tab) for x <= 0 or NaN, without a branch: the range ends as selects, and below them the
+// same operations (x is clamped where a select takes the result anyway; the exponent goes straight
+// into the high word, since ki << 47 has no bit below 32).
+__device__ __forceinline__ float qmh_expf_nonpos(float x, const uint64_t *tab) {
+    const double inv_ln2_n = 0x1.71547652b82fep+0 * 32.0, shift = 0x1.8p+52;
+    const double c0 = 0x1.c6af84b912394p-5 / 32.0 / 32.0 / 32.0;
+    const double c1 = 0x1.ebfce50fac4f3p-3 / 32.0 / 32.0;
+    const double c2 = 0x1.62e42ff0c52d6p-1 / 32.0;
+    const double xd = (double)fmaxf(x, -128.0f);
+    const double ks = __builtin_fma(inv_ln2_n, xd, shift);
+    const uint32_t ki = (uint32_t)__double2loint(ks);
+    const double r = __builtin_fma(inv_ln2_n, xd, -(ks - shift));
+    const uint64_t t = tab[ki % 32];
+    const double s = __hiloint2double((int)((uint32_t)(t >> 32) + (ki << 15)), (int)(uint32_t)t);
+    const double z = __builtin_fma(c0, r, c1), r2 = r * r;
+    double y = __builtin_fma(c2, r, 1.0);
+    y = __builtin_fma(z, r2, y) * s;
+    const float f = x < -0x1.9fe368p6f ? 0.0f : (float)y;
+    return x != x ? x + x : f;
+}
 // --------------------------------------------------------------------------- reductions
 
 template <int CTRL>

@@ -1206,89 +1206,73 @@ __global__ __launch_bounds__(QMH_WG) void k_pf_scores(const float *__restrict__ 
         if (k < np && t <= pos0 + p0 + k) att[((size_t)h * P + p0 + k) * max_seq + t] = s[k] * scale;
 }
 
-// The same scores blocked in registers: a workgroup takes 64 tokens x 64 positions, each thread
-// 4 tokens x 4 positions (16 chains). The query and K^T tiles ([HD][64] each) are staged in LDS;
-// per dimension a thread reads 4 query and 4 key values (two 16-byte LDS reads) for 32 VALU
-// operations. (One token x 16 positions per lane needs 16 LDS values per 32 operations, which
-// saturates the LDS return path before the VALU.) Same chains: s = +0, s = s + q[d] * k[d] over d
-// in order, then s * scale.
+// The same scores with the products from MFMAs, for head_dim 128, 64 and 48: v_mfma_f32_16x16x1_4b_f32
+// with a zero accumulator is 1024 correctly rounded products q[d] * k[d] (16 tokens x 4 x 16 positions;
+// checked on the device over every exponent, subnormals and special values included), and the VALU
+// adds them to the chains: s = +0, s = s + q[d] * k[d] over d in order, then s * scale. (A product of
+// -0 may come out as +0: a chain is never -0, so the sum is the same.) The f32 MFMA runs on the VALU's
+// units at the rate of its multiplies, but it takes one register each of query and key per 1024 products,
+// straight from memory, where register blocking on the VALU (4 x 4 per thread) read 32 bytes of LDS per
+// 16 products and filled the LDS return path. One wave per tile of 16 tokens x 64 positions; a workgroup's
+// 4 waves take 4 consecutive token tiles of the same positions, whose keys they share in L1. Timed, us,
+// register blocking -> this: 512 tokens, 32 heads x 128 dimensions 33 -> 29; a 1901-token prompt of 32
+// heads x 64, per 512-token pass, 49 -> 46 (two VALU operations per pair and dimension at two waves per
+// SIMD would be 14 and 24; the score writes are 12 of the 46). 32 x 64 tiles, and queries in scalar
+// registers (8 tokens x 128 positions per wave), took 36-39 at the first shape.
 template <int HD>
-__global__ __launch_bounds__(QMH_WG) void k_pf_scores_rb(const float *__restrict__ Q, const float *__restrict__ Kt,
-                                                         float *att, int P, int pos0, int n_heads, int n_kv,
-                                                         int max_seq, float scale) {
-    // the dimensions pass in phases of DP: 32 KB of LDS per workgroup, so that five share a CU and
-    // the causal half of the tiles (1152 of 2048 at 512 tokens) runs in one round
-    constexpr int DP = HD < 64 ? HD : 64;
-    __shared__ __align__(16) float qs[DP * 64];  // [d][token]
-    __shared__ __align__(16) float ks[DP * 64];  // [d][position]
-    const int h = blockIdx.x, tid = threadIdx.x;
-    const int p0 = blockIdx.y * 64, c0 = blockIdx.z * 64;
-    if (c0 > pos0 + min(p0 + 63, P - 1)) return;  // the whole tile is past every token (uniform)
+__global__ __launch_bounds__(QMH_WG, 4) void k_pf_scores_m(const float *__restrict__ Q, const float *__restrict__ Kt,
+                                                           float *att, int P, int pos0, int n_heads, int n_kv,
+                                                           int max_seq, float scale) {
+    constexpr int DG = 8;  // dimensions per register set; the next set loads while one is used
+    static_assert(HD % (2 * DG) == 0, "whole pairs of sets");
+    const int h = blockIdx.x, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63;
+    const int p0 = blockIdx.y * 64 + 16 * wave, c0 = blockIdx.z * 64;
+    if (p0 >= P || c0 > pos0 + min(p0 + 15, P - 1)) return;  // past the prompt, or past every token (whole wave)
     const int kvh = h / (n_heads / n_kv);
-    const int tg = tid >> 4, pg = tid & 15;  // tokens 4*tg .. +3, positions 4*pg .. +3
-    float s[4][4];
+    const int p = p0 + (l & 15), pc = p < P ? p : P - 1, tc = min(c0 + l, max_seq - 1);
+    const float *q = Q + ((size_t)pc * n_heads + h) * HD;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(Kt + (size_t)kvh * HD * max_seq), (short)0, (int)((uint32_t)HD * (uint32_t)max_seq * 4u), 0x00020000);
+    pf_v4f qv[2][DG / 4];
+    float kv[2][DG];
+    auto load = [&](int d0, int w) {
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+        for (int d = 0; d < DG / 4; d++) qv[w][d] = *(const pf_v4f *)(q + d0 + 4 * d);
 #pragma unroll
-        for (int b = 0; b < 4; b++) s[a][b] = 0.0f;
+        for (int d = 0; d < DG; d++) kv[w][d] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, tc * 4, (d0 + d) * max_seq * 4, 0));
+    };
+    float s[16];
+    pf_v16f z;
 #pragma unroll
-    for (int d0 = 0; d0 < HD; d0 += DP) {
-        if (d0) __syncthreads();  // the previous phase's reads are done
-        const float *kt = Kt + ((size_t)kvh * HD + d0) * max_seq;
+    for (int e = 0; e < 16; e++) s[e] = z[e] = 0.0f;
+    load(0, 0);
+#pragma unroll 1
+    for (int d0 = 0; d0 < HD; d0 += 2 * DG) {
 #pragma unroll
-        for (int k = 0; k < DP * 64 / QMH_WG; k++) {  // K^T rows, coalesced; positions past max_seq read the last
-            const int e = k * QMH_WG + tid, t = c0 + (e & 63);
-            ks[e] = kt[(size_t)(e >> 6) * max_seq + (t < max_seq ? t : max_seq - 1)];
-        }
-        const float *qh = Q + (size_t)h * HD + d0;
+        for (int w = 0; w < 2; w++) {
+            const int dn = d0 + (w + 1) * DG;
+            load(dn < HD ? dn : 0, w ^ 1);
+            // the next dimension's products go out before this one's are added
+            pf_v16f f[2];
+            auto mul = [&](int d) { f[d & 1] = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[w][d / 4][d % 4], kv[w][d], z, 0, 0, 0); };
+            mul(0);
 #pragma unroll
-        for (int k = 0; k < DP * 64 / 4 / QMH_WG; k++) {  // 4 dimensions of one token per thread; tokens past P read the last
-            const int e = k * QMH_WG + tid, tok = e & 63, d4 = e >> 6;
-            const int p = p0 + tok < P ? p0 + tok : P - 1;
-            const float4 v = *(const float4 *)(qh + (size_t)p * n_heads * HD + 4 * d4);
-            qs[(4 * d4) * 64 + tok] = v.x;
-            qs[(4 * d4 + 1) * 64 + tok] = v.y;
-            qs[(4 * d4 + 2) * 64 + tok] = v.z;
-            qs[(4 * d4 + 3) * 64 + tok] = v.w;
-        }
-        __syncthreads();
-        // dimension d + KA's values are read while dimension d is used. An empty asm per step pins
-        // the chains and the reads to their step: otherwise the compiler hoists every read to the
-        // top and sinks the arithmetic (DP*8 live registers)
-        constexpr int KA = 2;
-        float4 qv[KA + 1], kv[KA + 1];
+            for (int d = 0; d < DG; d++) {
+                if (d + 1 < DG) mul(d + 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int d = 0; d < KA; d++) {
-            qv[d] = *(const float4 *)(qs + d * 64 + 4 * tg);
-            kv[d] = *(const float4 *)(ks + d * 64 + 4 * pg);
-        }
-#pragma unroll
-        for (int d = 0; d < DP; d++) {
-            if (d + KA < DP) {
-                qv[(d + KA) % (KA + 1)] = *(const float4 *)(qs + (d + KA) * 64 + 4 * tg);
-                kv[(d + KA) % (KA + 1)] = *(const float4 *)(ks + (d + KA) * 64 + 4 * pg);
+                for (int e = 0; e < 16; e++) s[e] = s[e] + f[d & 1][e];
+                __builtin_amdgcn_sched_barrier(0);
             }
-            const float4 a4 = qv[d % (KA + 1)], b4 = kv[d % (KA + 1)];
-            const float qa[4] = {a4.x, a4.y, a4.z, a4.w}, kb[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++) s[a][b] = s[a][b] + qa[a] * kb[b];
-            asm volatile("" : "+v"(s[0][0]), "+v"(s[0][1]), "+v"(s[0][2]), "+v"(s[0][3]), "+v"(s[1][0]), "+v"(s[1][1]),
-                         "+v"(s[1][2]), "+v"(s[1][3]), "+v"(s[2][0]), "+v"(s[2][1]), "+v"(s[2][2]), "+v"(s[2][3]),
-                         "+v"(s[3][0]), "+v"(s[3][1]), "+v"(s[3][2]), "+v"(s[3][3])::"memory");
         }
     }
+    // element 4*b + e: token 4*(l/16) + e, position 16*b + l%16
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int p = p0 + 4 * tg + a;
-        if (p >= P) continue;
-        float *row = att + ((size_t)h * P + p) * max_seq;
+    for (int e = 0; e < 4; e++) {
+        const int pt = p0 + 4 * (l >> 4) + e;
+        float *row = att + ((size_t)h * P + pt) * max_seq + c0 + (l & 15);
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int t = c0 + 4 * pg + b;
-            if (t <= pos0 + p) row[t] = s[a][b] * scale;
-        }
+        for (int b = 0; b < 4; b++)
+            if (pt < P && c0 + 16 * b + (l & 15) <= pos0 + pt) row[16 * b] = s[4 * b + e] * scale;
     }
 }
 
@@ -1320,50 +1304,98 @@ __global__ __launch_bounds__(QMH_WG) void k_pf_softmax(float *att, int P, int po
     for (int t = lane; t < n; t += 64) x[t] = qmh_expf(x[t] - m) * inv;
 }
 
-// k_pf_softmax with the row in registers (rows of up to 64*R positions): one range-checked load
-// per value, all issued at once; each exponential is computed once and kept for both the sum and
-// the probability (the same values k_pf_softmax computes twice). The serial fallback reads the
-// scores, which stay untouched until the final stores.
-template <int R>
+// k_pf_softmax with the row in registers (rows of up to 64*W*R positions, W waves per row): one
+// range-checked load per value, all issued at once; each exponential is computed once and kept for both
+// the sum and the probability (the same values k_pf_softmax computes twice). The exponentials take no
+// branch (qmh_expf_nonpos) and their table from LDS, so a lane's R of them overlap; with the branches of
+// qmh_expf each waited for the one before. Timed, us per 512-token pass of 32 heads, before ->
+// after: rows up to 512 31 -> 14, up to 1901 140 -> 41 (one wave per row recomputing each exponential); the
+// serial sum, below, was most of it.
+template <int R, int W>
 __global__ __launch_bounds__(QMH_WG) void k_pf_softmax_r(float *att, int P, int pos0, int max_seq) {
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // uniform: a scalar resource
-    const int h = blockIdx.x, p = blockIdx.y * (QMH_WG / 64) + wave, lane = threadIdx.x & 63;
-    if (p >= P) return;  // the whole wave
-    const int n = pos0 + p + 1;
-    float *x = att + ((size_t)h * P + p) * max_seq;
+    __shared__ uint64_t tab[32];
+    __shared__ float redf[4];
+    __shared__ double redd[4];
+    constexpr int RW = 4 / W, LN = 64 * W;  // rows per workgroup, lanes per row
+    __shared__ float ex[W > 1 ? LN * R : 1];  // the exponentials, for the serial sum
+    const int tid = threadIdx.x;
+    const int rw = __builtin_amdgcn_readfirstlane(tid / LN);  // uniform per wave: a scalar resource
+    const int h = blockIdx.x, p = blockIdx.y * RW + rw, lane = tid % LN;
+    if (tid < 32) tab[tid] = qmh_exp2_tab[tid];
+    const int pc = p < P ? p : P - 1;
+    const int n = pos0 + pc + 1;
+    float *x = att + ((size_t)h * P + pc) * max_seq;
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, n * 4, 0x00020000);
     float xv[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) xv[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, (r * 64 + lane) * 4, 0, 0));
+    for (int r = 0; r < R; r++) xv[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, (r * LN + lane) * 4, 0, 0));
+    const float x0 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, 0, 0, 0));
+    __syncthreads();
+    if (p >= P) return;  // W == 1: whole waves, and no barrier follows
     float m = -__builtin_inff();
 #pragma unroll
     for (int r = 0; r < R; r++)
-        if (r * 64 + lane < n) m = xv[r] > m ? xv[r] : m;
+        if (r * LN + lane < n) m = xv[r] > m ? xv[r] : m;
     m = qmh_wave_max(m);
-    const float x0 = __shfl(xv[0], 0);
+    if (W > 1) {
+        if ((tid & 63) == 0) redf[tid >> 6] = m;
+        __syncthreads();
+        m = redf[0];
+#pragma unroll
+        for (int w = 1; w < W; w++) m = fmaxf(m, redf[w]);
+    }
     if (x0 != x0) m = x0;  // the reference's scan starts from x[0]: a NaN there stays
     float e[R];
     double sum = 0.0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
         e[r] = 0.0f;
-        if (r * 64 < n) {  // uniform: rounds past the row cost nothing (rows are 1 .. 64*R long)
-            e[r] = qmh_expf(xv[r] - m);
-            if (r * 64 + lane < n) sum += (double)e[r];
+        if (r * LN < n) {  // uniform: rounds past the row cost nothing
+            e[r] = qmh_expf_nonpos(xv[r] - m, tab);
+            e[r] = r * LN + lane < n ? e[r] : 0.0f;  // + 0 leaves the sum as it is
+            sum += (double)e[r];
         }
     }
     sum = qmh_wave_sum_d(sum);
+    if (W > 1) {
+        if ((tid & 63) == 0) redd[tid >> 6] = sum;
+        __syncthreads();
+        sum = redd[0];
+#pragma unroll
+        for (int w = 1; w < W; w++) sum += redd[w];
+    }
     const double d = qmh_sum_slack(sum, n);
     float inv = qmh_recip_of_sum(sum - d);
-    if (inv != qmh_recip_of_sum(sum + d)) {  // uniform; serial sum as the reference
+    if (inv != qmh_recip_of_sum(sum + d)) {  // uniform over the row; serial sum as the reference
+        // every lane of a wave adds the row's exponentials in order, broadcast from the lanes that hold
+        // them (about 20 cycles each; one lane recomputing them took 140 ns each, 83 us for a row that
+        // most calls of 512 rows x 32 heads have one of in thirty)
         double ser = 0.0;
-        if (lane == 0)
-            for (int t = 0; t < n; t++) ser += (double)qmh_expf(x[t] - m);
-        inv = qmh_recip_of_sum(__shfl(ser, 0));
+        if (W > 1) {
+#pragma unroll
+            for (int r = 0; r < R; r++) ex[r * LN + lane] = e[r];
+            __syncthreads();
+        }
+#pragma unroll 1
+        for (int c = 0; c < n; c += 64) {
+            float v;
+            if (W > 1) {
+                v = ex[c + (tid & 63)];
+            } else {
+                v = e[0];
+#pragma unroll
+                for (int r = 1; r < R; r++) v = c == 64 * r ? e[r] : v;
+            }
+            const int nc = n - c < 64 ? n - c : 64;
+#pragma unroll 1
+            for (int i = 0; i < nc; i++)
+                ser += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
+        }
+        inv = qmh_recip_of_sum(ser);
     }
 #pragma unroll
     for (int r = 0; r < R; r++)
-        if (r * 64 + lane < n) x[r * 64 + lane] = e[r] * inv;
+        if (r * LN + lane < n) x[r * LN + lane] = e[r] * inv;
 }
 
 // out[token][h*hd + i] = +0 + p_0 v_0[i] + p_1 v_1[i] + ... in position order (src/model.c:147-154);
@@ -1470,185 +1502,156 @@ __global__ __launch_bounds__(QMH_WG) void k_pf_pv(const float *__restrict__ att,
         }
 }
 
-// The same P·V blocked in registers for head_dim 128 and 64: each thread extends 4 tokens x 2
-// columns (8 chains), a workgroup 2048/HD tokens. Per position a thread reads the 4 tokens'
-// probabilities (one 16-byte LDS read) and 2 V values (8 bytes) for 16 VALU operations, against 36
-// bytes for the same 16 with one column x 8 tokens per thread, which fills the LDS return path.
-// The chunks, the unmasked runs and the diagonal's selects are as in k_pf_pv.
+// The same P.V with the products from MFMAs, for head_dim 128, 64 and 48: v_mfma_f32_16x16x1_4b_f32 with a
+// zero accumulator gives the products p_t * v_t[i] (rounded as the reference rounds them, see
+// k_pf_scores_m) of 16 tokens x 32 columns at two positions, t + j in its first two 16x16 blocks and
+// t + 4 + j in the others; four of them (j = 0..3) hold 8 positions, and 64 VALU adds then extend the 8
+// chains of each lane position by position. Per 8 positions a wave loads one 16-byte piece of probabilities
+// and four V values per lane, with no LDS and no barrier. The number of chains bounds the parallelism: with
+// 32 columns per wave, 512 tokens x 32 heads x 64 columns are two waves per SIMD (64 columns per wave and
+// one position per MFMA left one, which issues VALU work at half the rate: 81 us where this takes 50).
+// Register blocking on the VALU (4 tokens x 2 columns per thread) read 24 bytes of LDS per 8 products;
+// probabilities in scalar registers waited for the scalar cache. Positions up to the first token's are
+// seen by every token; the last 15 extend only the chains of the tokens that see them (a select, never an
+// added zero: a NaN from V must not pass). Wo's input image (xc): the tile through LDS, then the
+// quantizer's steps. Timed, us, register blocking -> this: 512 tokens, 32 heads x 128 columns 44 -> 26; a
+// 1901-token prompt of 32 heads x 64, per 512-token pass, 98 -> 50.
 template <int HD>
-__global__ __launch_bounds__(QMH_WG) void k_pf_pv_rb(const float *__restrict__ att, const float *__restrict__ V,
-                                                     float *out, int P, int pos0, int n_heads, int n_kv, int max_seq,
-                                                     int8_t *xc, float *xd, int PP, int perm8) {
-    constexpr int T = 2048 / HD, VC = QMH_PF_VC;     // tokens per workgroup, positions per chunk
-    constexpr int VR = VC * HD / 4 / QMH_WG;          // float4 of V per thread per chunk
-    constexpr int PR = T * VC / QMH_WG;               // probabilities per thread per chunk
-    __shared__ __align__(16) float ps[VC * T];        // [t][token]
-    __shared__ __align__(16) float vs[VC * HD];       // [t][column]
-    // token groups by quadrant of blockIdx.y, the odd quadrants reversed: the workgroups that share
-    // a CU (y = g, g + ng/4, g + ng/2, g + 3ng/4 when all are resident at once) then carry equal
-    // work in sum (late groups see more positions)
-    const int ng = gridDim.y, q4 = ng / 4, gy = blockIdx.y;
-    const int grp = (ng % 4 == 0 && (gy / q4) % 2 == 1) ? (gy / q4) * q4 + (q4 - 1 - gy % q4) : gy;
-    const int h = blockIdx.x, p0 = grp * T, np = min(T, P - p0);
-    const int kvh = h / (n_heads / n_kv), kvd = HD * n_kv, tid = threadIdx.x;
-    const int tmax = pos0 + p0 + np;  // positions 0 .. tmax-1 are used by some token
-    const int tall = pos0 + p0 + 1;   // positions 0 .. tall-1 are used by every token of the group
-    const float *vbase = V + (size_t)kvh * HD;
-    pf_v4f vr[VR];  // a vector type: float4 copies became memcpys through a stack slot
-    float pr[PR];
-#define PV_RB_LOAD(C0)                                                                                       \
-    _Pragma("unroll") for (int k = 0; k < VR; k++) {                                                         \
-        const int e = k * QMH_WG + tid, t = e / (HD / 4), c4 = e % (HD / 4);                                 \
-        const int tc = (C0) + t < tmax ? (C0) + t : tmax - 1;                                                \
-        vr[k] = *(const pf_v4f *)(vbase + (size_t)tc * kvd + 4 * c4);                                        \
-    }                                                                                                        \
-    _Pragma("unroll") for (int k = 0; k < PR; k++) {                                                         \
-        const int e = k * QMH_WG + tid, kk = e / VC, t = (C0) + e % VC;                                      \
-        pr[k] = (kk < np && t <= pos0 + p0 + kk) ? att[((size_t)h * P + p0 + kk) * max_seq + t] : 0.0f;      \
-    }
-    const int tg = tid / (HD / 2), cg = tid % (HD / 2);  // tokens 4*tg .. +3, columns 2*cg, 2*cg + 1
-    float acc[4][2];
+__global__ __launch_bounds__(QMH_WG, 4) void k_pf_pv_m(const float *__restrict__ att, const float *__restrict__ V,
+                                                       float *out, int P, int pos0, int n_heads, int n_kv, int max_seq,
+                                                       int8_t *xc, float *xd, int PP, int perm8) {
+    constexpr int CG = (HD + 31) / 32;             // 32-column groups of a head
+    constexpr int CW = CG % 4 == 0 ? 4 : CG % 2 == 0 ? 2 : 1, TW = 4 / CW;  // waves: CW column groups x TW token groups
+    __shared__ __align__(16) float tile[4][16][36];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63, hi = l >> 5;
+    // token groups, the long ones first and the second half reversed, so that the workgroups a CU gets
+    // carry equal work in sum
+    const int G = gridDim.y, half = (G + 1) / 2, y = blockIdx.y;
+    const int grp = y < half ? G - 1 - y : y - half;
+    const int h = blockIdx.x / (CG / CW), c0 = ((blockIdx.x % (CG / CW)) * CW + wave % CW) * 32;
+    const int p0 = (grp * TW + wave / CW) * 16;
+    if (p0 >= P) return;  // the whole wave; no barrier follows
+    const int np = min(16, P - p0), kvh = h / (n_heads / n_kv), kvd = HD * n_kv;
+    const int tall = pos0 + p0 + 1, tmax = pos0 + p0 + np;  // positions seen by every token, by some token
+    const int pl = p0 + (l & 15), cl = c0 + (l & 31);
+    // resources: the head's probabilities, the kv head's V; what lies past them (4-position loads at the end
+    // of the last row, positions past max_seq) reads as 0 and is not used
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(att + (size_t)h * P * max_seq), (short)0, (int)((uint32_t)P * (uint32_t)max_seq * 4u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(V + (size_t)kvh * HD), (short)0, (int)(((uint32_t)max_seq * (uint32_t)kvd - (uint32_t)(kvh * HD)) * 4u), 0x00020000);
+    const uint32_t po = ((uint32_t)(pl < P ? pl : P - 1) * (uint32_t)max_seq + 4u * hi) * 4u;
+    const uint32_t vo = ((uint32_t)(cl < HD ? cl : 0) + 4u * hi * (uint32_t)kvd) * 4u;
+    const int vst = kvd * 4;
+    constexpr int NB = 3;  // sets of 8 positions: one used, two in flight
+    pf_v4u pr[NB];
+    float vr[NB][4];
+    auto load = [&](int t, int w) {
+        pr[w] = __builtin_amdgcn_raw_buffer_load_b128(rp, po, t * 4, 0);
 #pragma unroll
-    for (int a = 0; a < 4; a++) acc[a][0] = acc[a][1] = 0.0f;
-    PV_RB_LOAD(0)
-    for (int c0 = 0; c0 < tmax; c0 += VC) {
-        __syncthreads();
+        for (int j = 0; j < 4; j++) vr[w][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, vo, (t + j) * vst, 0));
+    };
+    float s[8];  // element 4*b + e: token row0 + e, column 16*b + l%16
+    pf_v16f z;
 #pragma unroll
-        for (int k = 0; k < VR; k++) {
-            const int e = k * QMH_WG + tid;
-            *(pf_v4f *)(vs + (e / (HD / 4)) * HD + 4 * (e % (HD / 4))) = vr[k];
-        }
+    for (int e = 0; e < 16; e++) z[e] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < PR; k++) {
-            const int e = k * QMH_WG + tid;
-            ps[(e % VC) * T + e / VC] = pr[k];
-        }
-        if (c0 + VC < tmax) {
-            PV_RB_LOAD(c0 + VC)
-        }
-        __syncthreads();
-        const int nt = min(VC, tmax - c0);
-        const int nall = min(nt, max(tall - c0, 0));  // positions of this chunk every token sees
-        const float *pp = ps + 4 * tg, *vp = vs + 2 * cg;
-        int t = 0;
-        for (; t + 4 <= nall; t += 4) {
-            float4 pa[4];
-            float2 vv[4];
+    for (int e = 0; e < 8; e++) s[e] = 0.0f;
+    const int row0 = 4 * (l >> 4);
+    auto group = [&](int w, int t0, bool diag) {
+        pf_v16f f[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                pa[u] = *(const float4 *)(pp + (t + u) * T);
-                vv[u] = *(const float2 *)(vp + (t + u) * HD);
-            }
+        for (int j = 0; j < 4; j++)
+            f[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(__uint_as_float(pr[w][j]), vr[w][j], z, 0, 0, 0);
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float pk[4] = {pa[u].x, pa[u].y, pa[u].z, pa[u].w};
+        for (int k = 0; k < 8; k++) {
+            const int kmin = t0 + k - (pos0 + p0);  // tokens >= kmin see the position
 #pragma unroll
-                for (int a = 0; a < 4; a++) {
-                    acc[a][0] = acc[a][0] + pk[a] * vv[u].x;
-                    acc[a][1] = acc[a][1] + pk[a] * vv[u].y;
-                }
+            for (int e = 0; e < 8; e++) {
+                const float nx = s[e] + f[k % 4][8 * (k / 4) + e];
+                s[e] = !diag || row0 + (e & 3) >= kmin ? nx : s[e];
             }
         }
-        for (; t < nt; t++) {
-            const float4 p4 = *(const float4 *)(pp + t * T);
-            const float2 v2 = *(const float2 *)(vp + t * HD);
-            const float pk[4] = {p4.x, p4.y, p4.z, p4.w};
-            const int kmin = c0 + t - (pos0 + p0);  // tokens kk >= kmin see position c0 + t
+    };
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const bool on = 4 * tg + a >= kmin;
-                const float n0 = acc[a][0] + pk[a] * v2.x, n1 = acc[a][1] + pk[a] * v2.y;
-                acc[a][0] = on ? n0 : acc[a][0];
-                acc[a][1] = on ? n1 : acc[a][1];
+    for (int w = 0; w < NB - 1; w++) load(8 * w, w);
+#pragma unroll 1
+    for (int t = 0; t < tmax; t += 8 * NB) {
+#pragma unroll
+        for (int w = 0; w < NB; w++) {
+            const int tw = t + 8 * w;
+            if (tw < tmax) {  // uniform
+                load(tw + 8 * (NB - 1), (w + NB - 1) % NB);
+                if (tw + 8 <= tall) group(w, tw, false);
+                else group(w, tw, true);
             }
         }
     }
+    if (!xc) {
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int kk = 4 * tg + a;
-        if (kk < np) {
-            float *o = out + (size_t)(p0 + kk) * n_heads * HD + h * HD + 2 * cg;
-            o[0] = acc[a][0];
-            o[1] = acc[a][1];
-        }
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (row0 + e < np && c0 + 16 * b + (l & 15) < HD)
+                    out[((size_t)(p0 + row0 + e) * n_heads + h) * HD + c0 + 16 * b + (l & 15)] = s[4 * b + e];
+        return;
     }
-    if (xc) {  // uniform
-        // Wo's input as its Q8_0 image (the quantizer's steps, src/quant.c:27-52): block b of a token
-        // is columns 32*(cg/16) .. +31 of the head, held by the 16 lanes of cg/16 (values 2j, 2j+1 of
-        // the block in lane j = cg % 16): amax over those lanes, the fp16 scale, the codes. Q4_0
-        // consumers take each 8-group as e0 e2 e4 e6 e1 e3 e5 e7: lane j's two codes are bytes j % 4
-        // and 4 + j % 4 of group j / 4.
-        const int j = cg & 15, b = h * (HD / 32) + (cg >> 4);
 #pragma unroll
-        for (int a = 0; a < 4; a++) {
-            const int kk = 4 * tg + a;
-            float m = 0.0f;
+    for (int b = 0; b < 2; b++)
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const float av = fabsf(acc[a][c]);
-                m = av > m ? av : m;
-            }
+        for (int e = 0; e < 4; e++) tile[wave][row0 + e][16 * b + (l & 15)] = s[4 * b + e];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // within the wave: LDS operations stay in order
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                const float t = __shfl_xor(m, o);
-                m = t > m ? t : m;
-            }
-            const float dd = qmh_h2f(qmh_f2h(qmh_div127(m)));
-            const float v4[4] = {acc[a][0], acc[a][1], 0.0f, 0.0f};
-            int q[4];
-            qmh_q8_codes4(v4, dd, qmh_rcp(dd), q);
-            const uint32_t c0 = (uint32_t)q[0] & 0xffu, c1 = (uint32_t)q[1] & 0xffu;
-            int8_t *blk = xc + ((size_t)b * PP + p0 + kk) * 32;
-            if (perm8) {
-                uint32_t w0 = c0 << (8 * (j & 3)), w1 = c1 << (8 * (j & 3));
-                w0 |= (uint32_t)__shfl_xor((int)w0, 1);
-                w1 |= (uint32_t)__shfl_xor((int)w1, 1);
-                w0 |= (uint32_t)__shfl_xor((int)w0, 2);
-                w1 |= (uint32_t)__shfl_xor((int)w1, 2);
-                if (kk < np && (j & 3) == 0) *(uint2 *)(blk + 8 * (j >> 2)) = make_uint2(w0, w1);
-            } else {
-                uint32_t w = (c0 | (c1 << 8)) << (16 * (j & 1));
-                w |= (uint32_t)__shfl_xor((int)w, 1);
-                if (kk < np && (j & 1) == 0) *(uint32_t *)(blk + 2 * j) = w;
-            }
-            if (kk < np && j == 0) xd[(size_t)b * PP + p0 + kk] = dd;
-        }
+    for (int r = 0; r < 2; r++) {  // 8 lanes per token, 4 values each: one block of 32
+        const int kk = 8 * r + (l >> 3);
+        const pf_v4f x = *(const pf_v4f *)&tile[wave][kk][4 * (l & 7)];
+        const float v4[4] = {x[0], x[1], x[2], x[3]};
+        pf_quant_block(v4, h * (HD / 32) + c0 / 32, kk < np ? 0x7fffffff : 0, p0 + kk, l & 7, xc, xd, PP, perm8);
     }
-#undef PV_RB_LOAD
 }
 
 extern "C" int qmh_launch_pf_attention(const float *Q, const float *Kt, const float *V, float *att, float *out, int P,
                                        int pos0, int n_heads, int n_kv, int hd, int max_seq, float scale, int8_t *xc,
                                        float *xd, int PP, int perm8, void *stream) {
     if (hd > 128 || hd % 4 || pos0 + P > max_seq || P < 1) return (int)hipErrorInvalidValue;
-    // the output's quantized image comes only from the register-blocked P.V (head_dim 128 or 64)
+    // the output's quantized image comes only from k_pf_pv_m (head_dim 128 or 64: whole blocks)
     if (xc && (!xd || (hd != 128 && hd != 64) || P > PP)) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
     const int ng = (P + QMH_PF_TOK - 1) / QMH_PF_TOK, nz = (pos0 + P + QMH_WG - 1) / QMH_WG;
-    const dim3 gt(n_heads, (P + 63) / 64, (pos0 + P + 63) / 64);
-    if (hd == 128)
-        hipLaunchKernelGGL(k_pf_scores_rb<128>, gt, dim3(QMH_WG), 0, s, Q, Kt, att, P, pos0, n_heads, n_kv, max_seq,
-                           scale);
-    else if (hd == 64)
-        hipLaunchKernelGGL(k_pf_scores_rb<64>, gt, dim3(QMH_WG), 0, s, Q, Kt, att, P, pos0, n_heads, n_kv, max_seq,
-                           scale);
-    else
-        hipLaunchKernelGGL(k_pf_scores, dim3(n_heads, ng, nz), dim3(QMH_WG), 0, s, Q, Kt, att, P, pos0, n_heads, n_kv,
-                           hd, max_seq, scale);
-    const dim3 gs(n_heads, (P + QMH_WG / 64 - 1) / (QMH_WG / 64));
     const int rlen = pos0 + P;  // the longest row
-    if (rlen <= 64 * 4) hipLaunchKernelGGL(k_pf_softmax_r<4>, gs, dim3(QMH_WG), 0, s, att, P, pos0, max_seq);
-    else if (rlen <= 64 * 8) hipLaunchKernelGGL(k_pf_softmax_r<8>, gs, dim3(QMH_WG), 0, s, att, P, pos0, max_seq);
-    else if (rlen <= 64 * 16) hipLaunchKernelGGL(k_pf_softmax_r<16>, gs, dim3(QMH_WG), 0, s, att, P, pos0, max_seq);
-    else hipLaunchKernelGGL(k_pf_softmax, gs, dim3(QMH_WG), 0, s, att, P, pos0, max_seq);
-    if (hd == 128)
-        hipLaunchKernelGGL(k_pf_pv_rb<128>, dim3(n_heads, (P + 15) / 16), dim3(QMH_WG), 0, s, att, V, out, P, pos0,
-                           n_heads, n_kv, max_seq, xc, xd, PP, perm8);
-    else if (hd == 64)
-        hipLaunchKernelGGL(k_pf_pv_rb<64>, dim3(n_heads, (P + 31) / 32), dim3(QMH_WG), 0, s, att, V, out, P, pos0,
-                           n_heads, n_kv, max_seq, xc, xd, PP, perm8);
+    const dim3 wg(QMH_WG);
+    // head_dim 48, 64, 128: products from MFMAs (a layer's V and a head's probabilities within 4 GiB buffer
+    // resources, queries read as float4s)
+    const bool mf = (hd == 128 || hd == 64 || hd == 48) && (uint64_t)max_seq * hd * n_kv * 4 < 0xffffffffull &&
+                    (uint64_t)P * max_seq * 4 < 0xffffffffull && ((uintptr_t)Q & 15) == 0;
+    if (xc && !mf) return (int)hipErrorInvalidValue;
+#define PF_HD(K_, G_, ...)                                                         \
+    do {                                                                           \
+        if (hd == 128) hipLaunchKernelGGL(K_<128>, G_, wg, 0, s, __VA_ARGS__);     \
+        else if (hd == 64) hipLaunchKernelGGL(K_<64>, G_, wg, 0, s, __VA_ARGS__);  \
+        else hipLaunchKernelGGL(K_<48>, G_, wg, 0, s, __VA_ARGS__);                \
+    } while (0)
+    if (mf)
+        PF_HD(k_pf_scores_m, dim3(n_heads, (P + 63) / 64, (rlen + 63) / 64), Q, Kt, att, P, pos0, n_heads, n_kv,
+              max_seq, scale);
     else
-        hipLaunchKernelGGL(k_pf_pv, dim3(n_heads, ng), dim3(QMH_WG), 0, s, att, V, out, P, pos0, n_heads, n_kv, hd,
-                           max_seq);
+        hipLaunchKernelGGL(k_pf_scores, dim3(n_heads, ng, nz), wg, 0, s, Q, Kt, att, P, pos0, n_heads, n_kv, hd,
+                           max_seq, scale);
+    // one wave per row up to 512 positions, four beyond, the fewest rounds that hold the longest row
+    const dim3 g1(n_heads, (P + 3) / 4), g4(n_heads, P);
+#define PF_SM(R_, W_, G_) hipLaunchKernelGGL((k_pf_softmax_r<R_, W_>), G_, wg, 0, s, att, P, pos0, max_seq)
+    if (rlen <= 64 * 2) PF_SM(2, 1, g1);
+    else if (rlen <= 64 * 4) PF_SM(4, 1, g1);
+    else if (rlen <= 64 * 8) PF_SM(8, 1, g1);
+    else if (rlen <= 256 * 4) PF_SM(4, 4, g4);
+    else if (rlen <= 256 * 8) PF_SM(8, 4, g4);
+    else if (rlen <= 256 * 16) PF_SM(16, 4, g4);
+    else hipLaunchKernelGGL(k_pf_softmax, g1, wg, 0, s, att, P, pos0, max_seq);
+#undef PF_SM
+    if (mf)
+        PF_HD(k_pf_pv_m, dim3(n_heads, hd == 128 ? (P + 15) / 16 : (P + 31) / 32), att, V, out, P, pos0, n_heads, n_kv, max_seq,
+              xc, xd, PP, perm8);
+    else
+        hipLaunchKernelGGL(k_pf_pv, dim3(n_heads, ng), wg, 0, s, att, V, out, P, pos0, n_heads, n_kv, hd, max_seq);
+#undef PF_HD
     return (int)hipGetLastError();
 }
