@@ -281,113 +281,122 @@ extern "C" int qmh_launch_rope(float *v, int64_t n_heads, int64_t head_dim, cons
 // gemm_nt in the scalar ISA's order (src/gemm_driver.h:7-28): per element, K is cut into
 // panels of 256 (QM_GEMM_KC, src/kernels.h:37); each panel is a serial fp32 sum from +0 (each
 // product rounded alone, then added) and the panel sums are added to C (from +0) in order.
-// A workgroup of 256 threads owns 32x32 outputs, each thread a 2x2 block (four chains). A and B
-// pass through LDS in slices of GN_KS values of k, stored k-major ([k][row], rows padded to 34 so
-// the transposing writes are conflict-free and the float2 reads aligned); per k a thread reads two
-// float2 (its rows' A, its columns' B: the wave's four row pairs are broadcast reads) for four
-// multiplies and four adds. The next slice's global loads are in flight while a slice is summed.
-// Elements past M, N or K are staged as 0 and never added or stored.
+// The products come from MFMAs: v_mfma_f32_16x16x1_4b_f32 with a zero accumulator is four 16x16 blocks of
+// correctly rounded products (checked on the device over every exponent, subnormals and special values
+// included), here 16 rows x 16 columns at four consecutive k, and 16 VALU adds then extend each lane's four
+// chains in k order. (A product of -0 may come out as +0: a chain is never -0, so the sum is the same.) What
+// bounds it: 32 + 33 cycles per 1024 products and SIMD (the f32 MFMA runs on the VALU's units), from two
+// waves per SIMD on; one wave issues VALU work at half the rate, so a wave takes only 256 outputs.
+// Operands: a wave loads 32 k of its 16 rows of A and of B, eight lanes to a row (128 contiguous bytes),
+// passes them through LDS of its own (a wave's LDS operations stay in order, so there is no barrier) and
+// reads back k + 4*b .. +3 in lanes 16*b .. +15, the next chunk already in flight behind it. Read from memory
+// in that shape, every lane of a load is another cache line, and the address units bound the kernel (131
+// cycles per 1024 products). Four MFMAs go out together: turning the 4 k per lane by lane swaps into
+// k + 4*j + b for one MFMA at a time costs about 20 cycles per swap. Timed, us, 2 x 2 outputs per thread from
+// LDS -> this: 64^3 3.8 -> 3.1, 100x100x1000 26 -> 18, 512^3 15.7 -> 11.2, 1000x1090x1500 129 -> 77, 1024^3 85 -> 52,
+// 2048^3 570 -> 350 (the products and adds alone: 250).
 #define QMH_GEMM_KC 256
-#define GN_T 32   // outputs per workgroup side
-#define GN_KS 128  // k per LDS slice (divides QMH_GEMM_KC; a multiple of 32)
-#define GN_NQ (GN_KS / 32)  // float4 loads per thread per operand and slice
-#define GN_LD 34  // LDS row stride (floats)
-template <bool VEC>
-__global__ __launch_bounds__(256) void k_gemm_nt(const float *__restrict__ A, const float *__restrict__ B,
-                                                 float *__restrict__ C, int64_t M, int64_t N, int64_t K) {
-    static_assert(QMH_GEMM_KC % GN_KS == 0 && GN_T * GN_KS == 4 * 256 * GN_NQ, "whole float4s per thread per slice");
-    __shared__ __align__(16) float As[GN_KS][GN_LD], Bs[GN_KS][GN_LD];
-    const int tid = threadIdx.x, r = tid >> 4, c = tid & 15;  // rows 2r, 2r+1; columns 2c, 2c+1
-    const int64_t i0 = (int64_t)blockIdx.y * GN_T, j0 = (int64_t)blockIdx.x * GN_T;
-    // staging: thread t loads row t/8 of the tile, k 32*q + 4*(t%8) .. +3 of the slice (q < GN_NQ),
-    // for A and for B
-    const int sr = tid >> 3, sk = 4 * (tid & 7);
-    const float *ar = A + (i0 + sr < M ? i0 + sr : 0) * K, *br = B + (j0 + sr < N ? j0 + sr : 0) * K;
-    const bool aon = i0 + sr < M, bon = j0 + sr < N;
-    // no branches, and the values past M, N or K are zeroed only when the slice is stored, so the
-    // loads stay in flight under the previous slice's sums (VEC: K % 4 == 0 and rows 16-byte
-    // aligned, so a thread's 4 values are all in the row or all past K)
-    float va[GN_NQ][4], vb[GN_NQ][4];
-    auto fetch = [&](const float *row, int64_t k0, float (&v)[GN_NQ][4]) {
+#define GN_KG 16  // k per group of four MFMAs
+#define GN_KS 32  // k per chunk (two groups; divides QMH_GEMM_KC)
+#define GN_LD 36  // LDS row stride (floats): 16-byte reads of 8 consecutive rows cover every bank
+typedef float gn_v16f __attribute__((ext_vector_type(16)));
+typedef float gn_v4f __attribute__((ext_vector_type(4), aligned(4)));
+typedef float gn_v4a __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256, 4) void k_gemm_nt(const float *__restrict__ A, const float *__restrict__ B,
+                                                    float *__restrict__ C, int64_t M, int64_t N, int64_t K) {
+    static_assert(QMH_GEMM_KC % GN_KS == 0 && GN_KS == 2 * GN_KG, "a panel is whole chunks of two groups");
+    __shared__ __align__(16) float lds[4][2][16 * GN_LD];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63;
+    const int64_t i0 = (int64_t)blockIdx.y * 32 + 16 * (wave >> 1), j0 = (int64_t)blockIdx.x * 32 + 16 * (wave & 1);
+    if (i0 >= M || j0 >= N) return;  // the whole wave; no barrier follows
+    const int r = l & 15, lr = l >> 3, lk = 4 * (l & 7);  // loads: rows lr and lr + 8, k lk .. +3 of the chunk
+    const float *ar[2], *br[2];
 #pragma unroll
-        for (int q = 0; q < GN_NQ; q++) {
-            const int64_t k = k0 + 32 * q + sk;
-            if (VEC) {
-                const float4 f = *(const float4 *)(row + (k < K ? k : 0));
-                v[q][0] = f.x, v[q][1] = f.y, v[q][2] = f.z, v[q][3] = f.w;
-            } else {
+    for (int h = 0; h < 2; h++) {
+        const int64_t i = i0 + lr + 8 * h, j = j0 + lr + 8 * h;
+        ar[h] = A + (i < M ? i : M - 1) * K + lk;
+        br[h] = B + (j < N ? j : N - 1) * K + lk;
+    }
+    const int nc = (int)((K + GN_KS - 1) / GN_KS), nf = (int)(K / GN_KS);  // chunks, whole ones
+    gn_v4f ga[2], gb[2];
+    // +0 past K: 0 * 0 adds +0, which changes no chain; past the last chunk nothing is loaded
+    auto gload = [&](int c) {
+        const int64_t o = (int64_t)c * GN_KS;
+        if (c < nf) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[q][j] = row[k + j < K ? k + j : K - 1];
-            }
+            for (int h = 0; h < 2; h++) ga[h] = *(const gn_v4f *)(ar[h] + o), gb[h] = *(const gn_v4f *)(br[h] + o);
+        } else if (c < nc) {
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const bool in = o + lk + k < K;
+                    ga[h][k] = in ? ar[h][o + k] : 0.0f;
+                    gb[h][k] = in ? br[h][o + k] : 0.0f;
+                }
         }
     };
-    float c00 = 0.0f, c01 = 0.0f, c10 = 0.0f, c11 = 0.0f;
-    float s00 = 0.0f, s01 = 0.0f, s10 = 0.0f, s11 = 0.0f;
-    fetch(ar, 0, va);
-    fetch(br, 0, vb);
-    for (int64_t k0 = 0; k0 < K; k0 += GN_KS) {
-        __syncthreads();  // the previous slice is consumed
+    float *la = lds[wave][0], *lb = lds[wave][1];
+    auto swrite = [&] {
 #pragma unroll
-        for (int q = 0; q < GN_NQ; q++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const bool in = k0 + 32 * q + sk + j < K;
-                As[32 * q + sk + j][sr] = aon && in ? va[q][j] : 0.0f;
-                Bs[32 * q + sk + j][sr] = bon && in ? vb[q][j] : 0.0f;
-            }
-        __syncthreads();
-        if (k0 + GN_KS < K) {  // uniform: the next slice's loads under this slice's sums
-            fetch(ar, k0 + GN_KS, va);
-            fetch(br, k0 + GN_KS, vb);
+        for (int h = 0; h < 2; h++) {
+            *(gn_v4a *)(la + (lr + 8 * h) * GN_LD + lk) = (gn_v4a)ga[h];
+            *(gn_v4a *)(lb + (lr + 8 * h) * GN_LD + lk) = (gn_v4a)gb[h];
         }
-        const int kn = K - k0 < GN_KS ? (int)(K - k0) : GN_KS;
-        if (kn == GN_KS) {
-            // groups of 8 k from two register sets: group g+1's reads go out before group g's
-            // sums (held there by the scheduling barriers)
-            float2 xa[2][8], xb[2][8];
-            auto rd = [&](int g, float2(&da)[8], float2(&db)[8]) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes read it
+    };
+    gn_v4a av, bv;
+    auto rd = [&](int g) {
+        av = *(const gn_v4a *)(la + r * GN_LD + 16 * g + 4 * (l >> 4));
+        bv = *(const gn_v4a *)(lb + r * GN_LD + 16 * g + 4 * (l >> 4));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes overwrite it
+    };
+    float s[4], c[4];
+    gn_v16f z, f[4];
 #pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    da[q] = *(const float2 *)&As[8 * g + q][2 * r];
-                    db[q] = *(const float2 *)&Bs[8 * g + q][2 * c];
-                }
-            };
-            auto sum = [&](const float2(&da)[8], const float2(&db)[8]) {
+    for (int e = 0; e < 16; e++) z[e] = 0.0f;
 #pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    s00 = s00 + da[q].x * db[q].x;
-                    s01 = s01 + da[q].x * db[q].y;
-                    s10 = s10 + da[q].y * db[q].x;
-                    s11 = s11 + da[q].y * db[q].y;
-                }
-            };
-            rd(0, xa[0], xb[0]);
+    for (int e = 0; e < 4; e++) s[e] = c[e] = 0.0f;
+    auto mul4 = [&] {
 #pragma unroll
-            for (int g = 0; g < GN_KS / 8; g++) {
-                if (g + 1 < GN_KS / 8) rd(g + 1, xa[(g + 1) & 1], xb[(g + 1) & 1]);
-                __builtin_amdgcn_sched_barrier(0);
-                sum(xa[g & 1], xb[g & 1]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            for (int k = 0; k < kn; k++) {
-                const float2 a2 = *(const float2 *)&As[k][2 * r], b2 = *(const float2 *)&Bs[k][2 * c];
-                s00 = s00 + a2.x * b2.x;
-                s01 = s01 + a2.x * b2.y;
-                s10 = s10 + a2.y * b2.x;
-                s11 = s11 + a2.y * b2.y;
-            }
-        }
-        if ((k0 + GN_KS) % QMH_GEMM_KC == 0 || k0 + GN_KS >= K) {  // a panel ends: C += its sums
-            c00 = c00 + s00, c01 = c01 + s01, c10 = c10 + s10, c11 = c11 + s11;
-            s00 = s01 = s10 = s11 = 0.0f;
+        for (int j = 0; j < 4; j++) f[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[j], bv[j], z, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add4 = [&] {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) s[e] = s[e] + f[j][4 * k + e];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    gload(0);
+    swrite();
+    gload(1);
+    rd(0);
+    int left = QMH_GEMM_KC / GN_KS;  // chunks to the panel's end
+#pragma unroll 1
+    for (int i = 0; i < nc; i++) {
+        mul4();
+        rd(1);     // each group is read under the adds of the one before it
+        swrite();  // chunk i is read: chunk i + 1 in its place
+        gload(i + 2);
+        add4();
+        mul4();
+        rd(0);
+        add4();
+        if (--left == 0 || i + 1 == nc) {  // a panel ends: C += its sums
+#pragma unroll
+            for (int e = 0; e < 4; e++) c[e] = c[e] + s[e], s[e] = 0.0f;
+            left = QMH_GEMM_KC / GN_KS;
         }
     }
-    const int64_t i = i0 + 2 * r, j = j0 + 2 * c;
-    if (i < M && j < N) C[i * N + j] = c00;
-    if (i < M && j + 1 < N) C[i * N + j + 1] = c01;
-    if (i + 1 < M && j < N) C[(i + 1) * N + j] = c10;
-    if (i + 1 < M && j + 1 < N) C[(i + 1) * N + j + 1] = c11;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int64_t i = i0 + 4 * (l >> 4) + e, j = j0 + r;
+        if (i < M && j < N) C[i * N + j] = c[e];
+    }
 }
 
 // C = 0 for K = 0 (the reference's zeroing with no panel to add), as a kernel: no memset node if the
@@ -404,11 +413,8 @@ extern "C" int qmh_launch_gemm_nt(const float *A, const float *B, float *C, int6
         hipLaunchKernelGGL(k_gemm_zero, dim3(grid_for(M * N)), dim3(256), 0, (hipStream_t)stream, C, M * N);
         return (int)hipGetLastError();
     }
-    dim3 grid((unsigned)((N + GN_T - 1) / GN_T), (unsigned)((M + GN_T - 1) / GN_T));
-    if ((K & 3) == 0 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0)
-        hipLaunchKernelGGL(k_gemm_nt<true>, grid, dim3(256), 0, (hipStream_t)stream, A, B, C, M, N, K);
-    else
-        hipLaunchKernelGGL(k_gemm_nt<false>, grid, dim3(256), 0, (hipStream_t)stream, A, B, C, M, N, K);
+    const dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32));
+    hipLaunchKernelGGL(k_gemm_nt, grid, dim3(256), 0, (hipStream_t)stream, A, B, C, M, N, K);
     return (int)hipGetLastError();
 }
 
