@@ -1212,12 +1212,14 @@ __global__ __launch_bounds__(QMH_WG) void k_pf_scores(const float *__restrict__ 
 // adds them to the chains: s = +0, s = s + q[d] * k[d] over d in order, then s * scale. (A product of
 // -0 may come out as +0: a chain is never -0, so the sum is the same.) The f32 MFMA runs on the VALU's
 // units at the rate of its multiplies, but it takes one register each of query and key per 1024 products,
-// straight from memory, where register blocking on the VALU (4 x 4 per thread) read 32 bytes of LDS per
-// 16 products and filled the LDS return path. One wave per tile of 16 tokens x 64 positions; a workgroup's
+// where register blocking on the VALU (4 x 4 per thread) read 32 bytes of LDS per 16 products and filled the
+// LDS return path. Keys come straight from memory; below 128 dimensions a wave's queries go through LDS of its
+// own, loaded as whole rows (read from memory by token, each lane of a load is another cache line: 46 us
+// where this takes 42); at 128 the longer start and 34 KB of LDS per workgroup cost what that saves (29 -> 31). One wave per tile of 16 tokens x 64 positions; a workgroup's
 // 4 waves take 4 consecutive token tiles of the same positions, whose keys they share in L1. Timed, us,
 // register blocking -> this: 512 tokens, 32 heads x 128 dimensions 33 -> 29; a 1901-token prompt of 32
-// heads x 64, per 512-token pass, 49 -> 46 (two VALU operations per pair and dimension at two waves per
-// SIMD would be 14 and 24; the score writes are 12 of the 46). 32 x 64 tiles, and queries in scalar
+// heads x 64, per 512-token pass, 49 -> 42 (two VALU operations per pair and dimension at two waves per
+// SIMD would be 14 and 24; the score writes are 12 of the 42). 32 x 64 tiles, and queries in scalar
 // registers (8 tokens x 128 positions per wave), took 36-39 at the first shape.
 template <int HD>
 __global__ __launch_bounds__(QMH_WG, 4) void k_pf_scores_m(const float *__restrict__ Q, const float *__restrict__ Kt,
@@ -1225,12 +1227,24 @@ __global__ __launch_bounds__(QMH_WG, 4) void k_pf_scores_m(const float *__restri
                                                            int max_seq, float scale) {
     constexpr int DG = 8;  // dimensions per register set; the next set loads while one is used
     static_assert(HD % (2 * DG) == 0, "whole pairs of sets");
+    constexpr bool QL = HD < 128;  // queries through LDS
     const int h = blockIdx.x, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63;
     const int p0 = blockIdx.y * 64 + 16 * wave, c0 = blockIdx.z * 64;
     if (p0 >= P || c0 > pos0 + min(p0 + 15, P - 1)) return;  // past the prompt, or past every token (whole wave)
     const int kvh = h / (n_heads / n_kv);
-    const int p = p0 + (l & 15), pc = p < P ? p : P - 1, tc = min(c0 + l, max_seq - 1);
-    const float *q = Q + ((size_t)pc * n_heads + h) * HD;
+    const int tc = min(c0 + l, max_seq - 1);
+    const float *q = Q + ((size_t)min(p0 + (l & 15), P - 1) * n_heads + h) * HD;
+    if (QL) {  // the wave's queries, whole rows at a time
+        __shared__ __align__(16) float qs[QL ? 4 : 1][16][HD + 4];
+#pragma unroll
+        for (int i = 0; i < HD / 16; i++) {
+            const int r = (64 * i + l) / (HD / 4), d = 4 * ((64 * i + l) % (HD / 4));
+            *(pf_v4f *)&qs[wave][r][d] = *(const pf_v4f *)(Q + ((size_t)min(p0 + r, P - 1) * n_heads + h) * HD + d);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // within the wave: LDS operations stay in order
+        __builtin_amdgcn_wave_barrier();
+        q = qs[wave][l & 15];
+    }
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(Kt + (size_t)kvh * HD * max_seq), (short)0, (int)((uint32_t)HD * (uint32_t)max_seq * 4u), 0x00020000);
     pf_v4f qv[2][DG / 4];
     float kv[2][DG];
