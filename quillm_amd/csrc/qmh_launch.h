@@ -106,11 +106,19 @@ int qmh_launch_attn_batch(const float *Q, const float *Kt, const float *V, long 
                           void *stream);
 /* ---- batched prefill (qmh_prefill.hip) ---- */
 enum { QMH_PF_STORE = 0, QMH_PF_ADD = 1, QMH_PF_QKV = 2, QMH_PF_SWIGLU = 3 };
-/* token counts up to this run the skinny matmul (every weight streamed once for all tokens), larger
- * ones the tiled matmul */
+/* which matmul runs P tokens: the skinny one (a 16-row group per workgroup, one workgroup per CU, every weight
+ * streamed once) or the tiled one. The skinny matmul's time grows with the terms, rows * P; the tiled one's is the
+ * length of its chains until the tiles fill the chip (both grow alike with the columns). Timed, us, skinny -> tiled:
+ * 32000 rows x 4096 columns 39 -> 32 at 8 tokens, 61 -> 33 at 16; 2 x 11008 (W1 | W3) x 4096 34 -> 36 at 8, 45 -> 36 at
+ * 16, 130 -> 40 at 64; 12288 x 4096 26 -> 32 at 16, 39 -> 32 at 32; 2 x 5632 x 2048 18 -> 19 at 16, 25 -> 19 at 32; 4096
+ * rows stay ahead in the skinny one up to 64 tokens (59 -> 63). Below 8 tokens only the skinny one (and the
+ * multi-token matvec) is used, past QMH_PF_SKINNY_P only the tiled one. */
 #ifndef QMH_PF_SKINNY_P
 #define QMH_PF_SKINNY_P 64
 #endif
+static inline int qmh_pf_tiled(int P, int rows, int il) {
+    return P > QMH_PF_SKINNY_P || (P >= 8 && (long long)P * rows * (il ? 2 : 1) >= 300000);
+}
 typedef struct {
     /* weight: tiled codes/scales as for the matvec; il: interleaved W1 | W3 tiles */
     int dtype;
@@ -130,7 +138,7 @@ typedef struct {
     float eps;
     /* epilogue: out0 row-major [P][ld0]; QKV: q -> out0, k -> out1 ([kvd][max_seq]), v -> out2 */
     int epi;
-    /* SWIGLU through the tiled matmul (P > QMH_PF_SKINNY_P): with qxc set, the output is written only as the next
+    /* SWIGLU through the tiled matmul (qmh_pf_tiled): with qxc set, the output is written only as the next
      * matmul's Q8_0 image, codes [nb][PP][32] (Q4_0 order when qperm8) and scales [nb][PP], instead of
      * out0 (the quantization the launcher would run on it, bit for bit) */
     int8_t *qxc;

@@ -377,7 +377,7 @@ __device__ __forceinline__ void pf_store(const qmh_pf_args &a, int row, int p, f
     }
 }
 
-// ---- tiled matmul (more than QMH_PF_SKINNY_P tokens)
+// ---- tiled matmul (qmh_pf_tiled says when)
 //
 // A workgroup owns RT 32-row tiles x TT 32-token tiles, one (row tile, token tile) pair per wave, and
 // takes all blocks in order. IL (W1 | W3): the first RT/2 row tiles are W1 rows, the others the same
@@ -699,7 +699,7 @@ __global__ __launch_bounds__(64 * RT * TT, 4) void k_pf_gemm(qmh_pf_args a) {
     if (p < a.P && hi == 0) a.qxd[(size_t)b * a.PP + p] = dd;
 }
 
-// Skinny matmul for decode-sized batches (P <= 16*TT tokens, TT <= 4): one workgroup per 16-row group
+// Skinny matmul for decode-sized batches (P <= 16*TT tokens, TT <= 4; qmh_pf_tiled says when): one workgroup per 16-row group
 // streams every block of its rows once for all tokens. The blocks pass in rounds of as many as
 // fit the LDS budget at this P: wave w takes blocks base + 8j + w in batches of PD (each batch's
 // loads all in flight, no barrier inside a round), takes each block's exact int32 dot for TT
@@ -1059,8 +1059,8 @@ extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
     if (a->PP % 128 || a->P > a->PP || a->P < 1 || a->nb < 1) return (int)hipErrorInvalidValue;
     if ((a->epi == QMH_PF_SWIGLU) != (a->il != 0)) return (int)hipErrorInvalidValue;
     if (a->dtype != QMH_Q4 && a->dtype != QMH_Q8) return (int)hipErrorInvalidValue;
-    // the image output exists only in the tiled matmul's SwiGLU epilogue (more than QMH_PF_SKINNY_P tokens)
-    if (a->qxc && (a->epi != QMH_PF_SWIGLU || !a->qxd || a->P <= QMH_PF_SKINNY_P)) return (int)hipErrorInvalidValue;
+    // the image output exists only in the tiled matmul's SwiGLU epilogue
+    if (a->qxc && (a->epi != QMH_PF_SWIGLU || !a->qxd || !qmh_pf_tiled(a->P, a->rows, a->il))) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
     if (a->xf && (a->nxf < 1 || a->nxf > 32 * a->nb || a->ldxf < a->nxf)) return (int)hipErrorInvalidValue;
     // the multi-token matvec when one tile's terms fit its LDS with the records. It quantizes a plain
@@ -1107,7 +1107,7 @@ extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
 #undef BMV_GO
         return (int)hipGetLastError();
     }
-    if (a->P <= QMH_PF_SKINNY_P) {  // decode-sized batches: the skinny matmul streams every weight once
+    if (!qmh_pf_tiled(a->P, a->rows, a->il)) {  // decode-sized batches: the skinny matmul streams every weight once
         const dim3 g((a->rows + 15) / 16);
         const int nm = a->il ? 2 : 1;
         const size_t lds = (size_t)sk_round(a->nb, nm, a->P) * nm * 16 * a->P * sizeof(float);
@@ -1140,19 +1140,23 @@ extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
     // 2 x 2 where 4 x 2 would leave half of the CUs idle or more (timed, us, 4 x 2 -> 2 x 2: 4096x11008 at
     // 96 tokens, 64 workgroups, 82 -> 66; 2048x5632 at 512, 128, 47 -> 39; 4096x4096 at 300, 160,
     // 36.7 -> 37.8) and for W1 | W3, whose 64-slot tiles it reads whole (4096 columns: 197 -> 186; 2048:
-    // 59 -> 60), both with the loads two stages ahead.
+    // 59 -> 60), both with the loads two stages ahead. Up to 32 tokens 2 x 1, which has no second token
+    // tile to compute for nothing (2 x 2 -> 2 x 1: 32000x4096 36 -> 33, W1 | W3 40 -> 36, 12288x4096
+    // 34 -> 32).
     const int tg = (a->P + 63) / 64, g4 = tg * ((a->rows + 127) / 128);
-#define PG_LAUNCH(IL_, RT_, DEEP_, ROWS_)                                                                                \
-    do {                                                                                                                 \
-        const dim3 g(tg, (a->rows + (ROWS_)-1) / (ROWS_));                                                               \
-        if (a->dtype == QMH_Q4)                                                                                          \
-            hipLaunchKernelGGL((k_pf_gemm<QMH_Q4, IL_, RT_, 2, DEEP_>), g, dim3(128 * RT_), 0, s, *a);                \
-        else                                                                                                             \
-            hipLaunchKernelGGL((k_pf_gemm<QMH_Q8, IL_, RT_, 2, DEEP_>), g, dim3(128 * RT_), 0, s, *a);                \
+#define PG_LAUNCH(IL_, RT_, TT_, DEEP_, ROWS_)                                                                \
+    do {                                                                                                      \
+        const dim3 g((a->P + 32 * (TT_)-1) / (32 * (TT_)), (a->rows + (ROWS_)-1) / (ROWS_));                  \
+        if (a->dtype == QMH_Q4)                                                                               \
+            hipLaunchKernelGGL((k_pf_gemm<QMH_Q4, IL_, RT_, TT_, DEEP_>), g, dim3(64 * RT_ * TT_), 0, s, *a); \
+        else                                                                                                  \
+            hipLaunchKernelGGL((k_pf_gemm<QMH_Q8, IL_, RT_, TT_, DEEP_>), g, dim3(64 * RT_ * TT_), 0, s, *a); \
     } while (0)
-    if (a->il) PG_LAUNCH(true, 2, 1, 32);
-    else if (g4 <= 128) PG_LAUNCH(false, 2, 1, 64);
-    else PG_LAUNCH(false, 4, 0, 128);
+    if (a->il && a->P <= 32) PG_LAUNCH(true, 2, 1, 1, 32);
+    else if (a->il) PG_LAUNCH(true, 2, 2, 1, 32);
+    else if (a->P <= 32) PG_LAUNCH(false, 2, 1, 1, 64);
+    else if (g4 <= 128) PG_LAUNCH(false, 2, 2, 1, 64);
+    else PG_LAUNCH(false, 4, 2, 0, 128);
 #undef PG_LAUNCH
     return (int)hipGetLastError();
 }

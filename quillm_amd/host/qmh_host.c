@@ -406,7 +406,7 @@ struct qmh_model {
     int pf_ok, pf_cap, pf_pp;
     int32_t *d_pf_tok, *h_pf_tok;
     float *d_pf_x, *d_pf_xb, *d_pf_q, *d_pf_hb, *d_pf_att, *d_pf_logits, *d_pf_xd;
-    int8_t *d_pf_xc2; /* W2's input image, written by W1|W3's epilogue past QMH_PF_SKINNY_P tokens */
+    int8_t *d_pf_xc2; /* W2's input image, written by W1|W3's epilogue in the tiled matmul */
     float *d_pf_xd2;
     int8_t *d_pf_xc;
 };
@@ -1130,9 +1130,8 @@ static int pf_layer(qmh_model *m, int l, int P, int pos, const pf_seqs *bt, hipS
     a.epi = QMH_PF_SWIGLU;
     a.out0 = m->d_pf_hb;
     a.ld0 = H;
-    /* past the skinny matmul's token counts (the tiled matmul) hb is written only as W2's quantized
-     * image */
-    const int hb_image = P > QMH_PF_SKINNY_P;
+    /* from the tiled matmul hb is written only as W2's quantized image */
+    const int hb_image = qmh_pf_tiled(P, H, 1);
     if (hb_image) {
         a.qxc = m->d_pf_xc2;
         a.qxd = m->d_pf_xd2;

@@ -99,3 +99,16 @@ def test_nonfinite_scales(gpu, monkeypatch, where, vocab, wt):
 
     with model(gpu, 72, 200, 6, 2, vocab, 256, wt, edit) as m:
         check(m, monkeypatch, 70, vocab)
+
+
+# both sides of the rule that takes 8 to 64 tokens to the tiled matmul (300000 rows x tokens), for the output
+# (row counts that end inside tiles) and for W1 | W3, whose input image to W2 changes with it; one and two
+# token tiles
+@pytest.mark.parametrize("wt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("hidden,vocab,P", [(200, 37501, 7), (200, 37500, 8), (200, 37499, 8), (200, 9376, 32),
+                                            (200, 9376, 31), (200, 9091, 33), (4688, 300, 32), (4687, 300, 32),
+                                            (2381, 300, 63), (2380, 300, 63), (2344, 4688, 64)])
+def test_few_token_rule(gpu, monkeypatch, hidden, vocab, P, wt):
+    print(f"case {hidden} {vocab} {P} {wt}", flush=True)
+    with model(gpu, 72, hidden, 6, 2, vocab, 128, wt) as m:
+        check(m, monkeypatch, P, vocab)
