@@ -398,9 +398,10 @@ __device__ __forceinline__ void pf_store(const qmh_pf_args &a, int row, int p, f
 //
 // Operands pass through LDS in stages of PG_KB blocks, two buffers: a thread's pieces of stage i + 2
 // (+ DEEP) are loaded to registers during stage i and written when stage i has been read. The loads'
-// offsets are fixed per thread (buffer loads, the block in the scalar offset; the resource's size
-// zeroes what lies past the matrix), and the barrier waits for LDS only, so loads stay in flight
-// across it. Q4_0 codes are written as 16*(q - 8) (two operations per four codes; a chain of 16 x the
+// offsets are fixed per thread (buffer loads, the block in the scalar offset, which a buffer's range check
+// need not cover). The stages run past the last block, in a last stage that is not whole and in those
+// loaded ahead: these load the last block again, so that every address lies in the matrix, and what they
+// hold is never multiplied. The barrier waits for LDS only, so loads stay in flight across it. Q4_0 codes are written as 16*(q - 8) (two operations per four codes; a chain of 16 x the
 // terms is 16 x the reference's chain exactly, so one multiply by 1/16 ends it: no term is below
 // 2^-48 or above 2^52). In LDS each half block of every row (or token) is contiguous over the rows,
 // which has no bank conflicts; the four fp16 scales of a row sit side by side, and the scale product of
@@ -466,8 +467,11 @@ __global__ __launch_bounds__(64 * RT * TT, 4) void k_pf_gemm(qmh_pf_args a) {
         bx = (lin >> 3) % gx;
     }
     const int rg0 = by * (IL ? NR / 2 : NR), t0 = bx * NTK, nb = a.nb;
-    const int row = tid % NR, j0 = tid / NR;    // A: row of the tile, blocks j0 + k*RS
-    const int tok = tid % NTK, q0 = tid / NTK;  // B: token, (half, block) q0 + k*TS
+    // A: row of the tile, blocks j0 + k*RS (a wave's lanes share j0)
+    static_assert(NR % 64 == 0, "whole waves per block of A");
+    const int row = tid % NR, j0 = wave * 64 / NR;
+    // B: token, (half, block) q0 + k*TS: a wave's lanes share the block, q0 / 2 + k*TS/2
+    const int tok = tid % NTK, q0 = tid / NTK, qb = wave * 64 / NTK / 2;
     // offsets from the workgroup's first slot; rows past the allocated ones read its first row
     const uint32_t slot_w = pf_slot0(a, rg0, 0);
     auto slot_of = [&](int r) {
@@ -483,8 +487,8 @@ __global__ __launch_bounds__(64 * RT * TT, 4) void k_pf_gemm(qmh_pf_args a) {
     const __amdgpu_buffer_rsrc_t rcb = rsrc(a.xc + (size_t)t0 * 32, ((size_t)nb * a.PP - t0) * 32);
     const __amdgpu_buffer_rsrc_t rcd = rsrc(a.xd + t0, ((size_t)nb * a.PP - t0) * 4);
     const uint32_t ast = (uint32_t)a.tile_r * CB, bst = (uint32_t)a.PP * 32;
-    const uint32_t va = slot_r * CB + j0 * ast, vw = (slot_r + j0 * a.tile_r) * 2;
-    const uint32_t vb = tok * 32 + (q0 & 1) * 16 + (q0 >> 1) * bst, vd = (uint32_t)(tok + q0 * a.PP) * 4;
+    const uint32_t va = slot_r * CB, vw = slot_r * 2, vb = tok * 32 + (q0 & 1) * 16, vd = tok * 4;
+    auto blk = [&](int b) { return (uint32_t)(b < nb ? b : nb - 1); };
     pf_v4u ra_[1 + DEEP][NA][AH], rb_[1 + DEEP][NB];
     uint32_t rw_[1 + DEEP][NA], rd_[1 + DEEP][ND];
     // stage of blocks b0.. into register set q, and from there to the LDS buffer at base
@@ -493,14 +497,18 @@ __global__ __launch_bounds__(64 * RT * TT, 4) void k_pf_gemm(qmh_pf_args a) {
         for (int k = 0; k < NA; k++) {
 #pragma unroll
             for (int h = 0; h < AH; h++)
-                ra_[q][k][h] = __builtin_amdgcn_raw_buffer_load_b128(rca, va + 16 * h, (b0 + k * RS) * ast, 0);
-            rw_[q][k] = __builtin_amdgcn_raw_buffer_load_b16(rcw, vw, (b0 + k * RS) * a.tile_r * 2, 0);
+                ra_[q][k][h] = __builtin_amdgcn_raw_buffer_load_b128(rca, va + 16 * h, blk(b0 + j0 + k * RS) * ast, 0);
+            rw_[q][k] = __builtin_amdgcn_raw_buffer_load_b16(rcw, vw, blk(b0 + j0 + k * RS) * (uint32_t)a.tile_r * 2, 0);
         }
 #pragma unroll
-        for (int k = 0; k < NB; k++) rb_[q][k] = __builtin_amdgcn_raw_buffer_load_b128(rcb, vb, (b0 + k * (TS / 2)) * bst, 0);
+        for (int k = 0; k < NB; k++)
+            rb_[q][k] = __builtin_amdgcn_raw_buffer_load_b128(rcb, vb, blk(b0 + qb + k * (TS / 2)) * bst, 0);
 #pragma unroll
-        for (int k = 0; k < ND; k++)
-            if (TS <= KB || wave * 64 / NTK < KB) rd_[q][k] = __builtin_amdgcn_raw_buffer_load_b32(rcd, vd, (b0 + k * TS) * a.PP * 4, 0);
+        for (int k = 0; k < ND; k++) {  // block q0 + k*TS: shared by a wave's lanes from 64 tokens on
+            const uint32_t o = blk(b0 + (NTK < 64 ? q0 : wave * 64 / NTK) + k * TS) * (uint32_t)a.PP * 4;
+            if (TS <= KB || wave * 64 / NTK < KB)
+                rd_[q][k] = __builtin_amdgcn_raw_buffer_load_b32(rcd, NTK < 64 ? vd + o : vd, NTK < 64 ? 0 : o, 0);
+        }
     };
     auto swrite = [&](uint32_t base, int q) {
 #pragma unroll
