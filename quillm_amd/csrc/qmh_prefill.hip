@@ -1257,14 +1257,14 @@ __global__ __launch_bounds__(QMH_WG, 4) void k_pf_scores_m(const float *__restri
         __builtin_amdgcn_wave_barrier();
         q = qs[wave][l & 15];
     }
-    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(Kt + (size_t)kvh * HD * max_seq), (short)0, (int)((uint32_t)HD * (uint32_t)max_seq * 4u), 0x00020000);
+    const float *kt = Kt + (size_t)kvh * HD * max_seq;  // a uniform row pointer per dimension, the lane's position clamped
     pf_v4f qv[2][DG / 4];
     float kv[2][DG];
     auto load = [&](int d0, int w) {
 #pragma unroll
         for (int d = 0; d < DG / 4; d++) qv[w][d] = *(const pf_v4f *)(q + d0 + 4 * d);
 #pragma unroll
-        for (int d = 0; d < DG; d++) kv[w][d] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, tc * 4, (d0 + d) * max_seq * 4, 0));
+        for (int d = 0; d < DG; d++) kv[w][d] = (kt + (size_t)(d0 + d) * max_seq)[(uint32_t)tc];
     };
     float s[16];
     pf_v16f z;
@@ -1560,20 +1560,29 @@ __global__ __launch_bounds__(QMH_WG, 4) void k_pf_pv_m(const float *__restrict__
     const int np = min(16, P - p0), kvh = h / (n_heads / n_kv), kvd = HD * n_kv;
     const int tall = pos0 + p0 + 1, tmax = pos0 + p0 + np;  // positions seen by every token, by some token
     const int pl = p0 + (l & 15), cl = c0 + (l & 31);
-    // resources: the head's probabilities, the kv head's V; what lies past them (4-position loads at the end
-    // of the last row, positions past max_seq) reads as 0 and is not used
-    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(att + (size_t)h * P * max_seq), (short)0, (int)((uint32_t)P * (uint32_t)max_seq * 4u), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(V + (size_t)kvh * HD), (short)0, (int)(((uint32_t)max_seq * (uint32_t)kvd - (uint32_t)(kvh * HD)) * 4u), 0x00020000);
-    const uint32_t po = ((uint32_t)(pl < P ? pl : P - 1) * (uint32_t)max_seq + 4u * hi) * 4u;
-    const uint32_t vo = ((uint32_t)(cl < HD ? cl : 0) + 4u * hi * (uint32_t)kvd) * 4u;
-    const int vst = kvd * 4;
+    // Resources of one set of 8 positions, t .. t + 7: the token group's probabilities from position t of its
+    // first row to the end of its last one, V from position t's row to the eighth's, or to the last of
+    // max_seq. The sets loaded ahead run past the last position, and a 4-position load past the last row's
+    // end: a range check on the lane's offset alone reads those as 0, and they are not used. So each set has
+    // its base in its resources (scalar arithmetic) and nothing in the scalar offset, which the check need not
+    // cover.
+    const float *pbase = att + ((size_t)h * P + p0) * max_seq, *vbase = V + (size_t)kvh * HD;
+    const uint32_t po = ((uint32_t)(pl < P ? l & 15 : np - 1) * (uint32_t)max_seq + 4u * hi) * 4u;
+    uint32_t vo[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) vo[j] = ((uint32_t)(cl < HD ? cl : 0) + (4u * hi + j) * (uint32_t)kvd) * 4u;
     constexpr int NB = 3;  // sets of 8 positions: one used, two in flight
     pf_v4u pr[NB];
     float vr[NB][4];
     auto load = [&](int t, int w) {
-        pr[w] = __builtin_amdgcn_raw_buffer_load_b128(rp, po, t * 4, 0);
+        const int n = t < max_seq ? (max_seq - t < 8 ? max_seq - t : 8) : 0;  // positions from t on, up to 8
+        const uint32_t pn = n ? ((uint32_t)np * (uint32_t)max_seq - (uint32_t)t) * 4u : 0u;
+        const uint32_t vn = n ? ((uint32_t)n * (uint32_t)kvd - (uint32_t)(kvh * HD)) * 4u : 0u;
+        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(pbase + t), (short)0, (int)pn, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vbase + (size_t)t * kvd), (short)0, (int)vn, 0x00020000);
+        pr[w] = __builtin_amdgcn_raw_buffer_load_b128(rp, po, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; j++) vr[w][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, vo, (t + j) * vst, 0));
+        for (int j = 0; j < 4; j++) vr[w][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, vo[j], 0, 0));
     };
     float s[8];  // element 4*b + e: token row0 + e, column 16*b + l%16
     pf_v16f z;
@@ -1645,10 +1654,9 @@ extern "C" int qmh_launch_pf_attention(const float *Q, const float *Kt, const fl
     const int ng = (P + QMH_PF_TOK - 1) / QMH_PF_TOK, nz = (pos0 + P + QMH_WG - 1) / QMH_WG;
     const int rlen = pos0 + P;  // the longest row
     const dim3 wg(QMH_WG);
-    // head_dim 48, 64, 128: products from MFMAs (a layer's V and a head's probabilities within 4 GiB buffer
-    // resources, queries read as float4s)
-    const bool mf = (hd == 128 || hd == 64 || hd == 48) && (uint64_t)max_seq * hd * n_kv * 4 < 0xffffffffull &&
-                    (uint64_t)P * max_seq * 4 < 0xffffffffull && ((uintptr_t)Q & 15) == 0;
+    // head_dim 48, 64, 128: products from MFMAs (16 rows of probabilities and 8 of V within 32-bit offsets,
+    // queries read as float4s)
+    const bool mf = (hd == 128 || hd == 64 || hd == 48) && max_seq < 1 << 26 && n_kv < 1 << 16 && ((uintptr_t)Q & 15) == 0;
     if (xc && !mf) return (int)hipErrorInvalidValue;
 #define PF_HD(K_, G_, ...)                                                         \
     do {                                                                           \

@@ -13,10 +13,14 @@ positions, and checked against its buffer's extent:
   * k_bt_attn                quillm_amd/csrc/qmh_batch.hip:129-219 (V chunks of 128 positions
                              clamped to position n-1, the scores and probabilities in LDS after the
                              staged V, LDS of BT_FC*128 + max_pos + 1 floats)
-  * qmh_launch_pf_attention  quillm_amd/csrc/qmh_prefill.hip:1461-1494, with k_pf_scores_rb<HD>
-                             (:1057-1130), k_pf_softmax_r<R> (:1169-1209) and k_pf_pv_rb<HD>
-                             (:1320-1459, the quadrant-reversed token groups and Wo's quantized
-                             image)
+  * qmh_launch_pf_attention  quillm_amd/csrc/qmh_prefill.hip, with k_pf_scores_m<HD> (16 x 64 tiles, queries
+                             in LDS below 128 dimensions, positions clamped to max_seq - 1),
+                             k_pf_softmax_r<R, W> (W waves per row, the exponentials in LDS for W > 1) and
+                             k_pf_pv_m<HD> (sets of 8 positions loaded two ahead, each with buffer
+                             resources of its own, the reversed second half of the token groups and Wo's
+                             quantized image). A buffer load is in bounds when its resource lies in the
+                             array and nothing but the lane's offset, which the range check covers, is
+                             added to the resource's base
 The batched caches are [n_layers][B][kvd * max_seq] (qmh_batch_create, kv_stride = kvd*max_seq,
 quillm_amd/host/qmh_host.c:1337): a sequence's index past its own stride would read the next
 sequence's cache (or, for the last one, past the allocation), so the checks hold each sequence
@@ -219,97 +223,117 @@ def test_batched_model_catches_a_sequence_leaving_its_cache():
 
 # ---------------------------------------------------------------------------- prefill tiles
 
-def pf_scores_rb(HD, nh, nkv, S, P, pos0, e):
-    """k_pf_scores_rb<HD> over grid (n_heads, ceil(P/64), ceil((pos0+P)/64)) x 256 threads."""
-    DP = HD if HD < 64 else 64
-    group, D = nh // nkv, nh * HD
-    tid = np.arange(WG)
-    tg, pg = tid >> 4, tid & 15
-    assert 2 * 4 * DP * 64 <= 64 * 1024
-    for p0 in range(0, P, 64):
+def pf_scores_m(HD, nh, nkv, S, P, pos0, e):
+    """k_pf_scores_m<HD> over grid (n_heads, ceil(P/64), ceil((pos0+P)/64)) x 4 waves."""
+    group, DG = nh // nkv, 8
+    l = np.arange(64)
+    if HD < 128:  # the wave's 16 queries as whole rows in LDS, HD + 4 floats apart
+        i = (np.arange(HD // 16)[:, None] * 64 + l[None, :]).ravel()
+        r, d = i // (HD // 4), 4 * (i % (HD // 4))
+        assert np.array_equal(np.sort(r * HD + d), np.arange(0, 16 * HD, 4)), "every float4 of 16 queries once"
+        inb("pf scores LDS", r * (HD + 4) + d + 3, 16 * (HD + 4))
+    else:
+        r, d = l & 15, HD - 4
+    d0 = np.arange(0, HD, 2 * DG)  # sets of DG dimensions; the one after the last reads the first again
+    dn = np.concatenate([d0 + DG, np.where(d0 + 2 * DG < HD, d0 + 2 * DG, 0)])
+    assert dn.max() + DG <= HD
+    for p0 in range(0, P, 16):
         for c0 in range(0, pos0 + P, 64):
-            if c0 > pos0 + min(p0 + 63, P - 1):
+            if c0 > pos0 + min(p0 + 15, P - 1):
                 continue
+            tc = np.minimum(c0 + l, S - 1)
             for h in range(nh):
-                kvh = h // group
-                for d0 in range(0, HD, DP):
-                    ek = (np.arange(DP * 64 // WG)[:, None] * WG + tid[None, :]).ravel()
-                    inb("pf ks LDS", ek, DP * 64)
-                    t = c0 + (ek & 63)
-                    inb("pf K", (kvh * HD + d0) * S + (ek >> 6) * S + np.minimum(t, S - 1), e.K)
-                    eq = (np.arange(DP * 64 // 4 // WG)[:, None] * WG + tid[None, :]).ravel()
-                    tok, d4 = eq & 63, eq >> 6
-                    p = np.minimum(p0 + tok, P - 1)
-                    inb("pf Q", h * HD + d0 + p * D + 4 * d4 + 3, P * D)
-                    inb("pf qs LDS", (4 * d4 + 3) * 64 + tok, DP * 64)
-                    inb("pf qs/ks reads", (DP - 1) * 64 + 4 * np.maximum(tg, pg) + 3, DP * 64)
-                for a in range(4):
-                    p = p0 + 4 * tg + a
+                inb("pf Q", (np.minimum(p0 + r, P - 1) * nh + h) * HD + d + 3, P * nh * HD)
+                for dd in (0, HD - 1):
+                    inb("pf K", ((h // group) * HD + dd) * S + tc, e.K)
+                for el in range(4):
+                    pt = p0 + 4 * (l >> 4) + el
                     for b in range(4):
-                        t = c0 + 4 * pg + b
-                        on = (p < P) & (t <= pos0 + p)
-                        inb("pf att", ((h * P + p) * S + t)[on], nh * P * S)
+                        t = c0 + 16 * b + (l & 15)
+                        on = (pt < P) & (t <= pos0 + pt)
+                        inb("pf att", ((h * P + pt) * S + t)[on], nh * P * S)
 
 
 def pf_softmax(nh, S, P, pos0):
-    """k_pf_softmax_r<R> (rows up to 64R) or k_pf_softmax: row (head, token) of n = pos0+p+1."""
+    """k_pf_softmax_r<R, W> (rows up to 64*W*R) or k_pf_softmax: row (head, token) of n = pos0+p+1."""
     rlen = pos0 + P
-    R = 4 if rlen <= 256 else 8 if rlen <= 512 else 16 if rlen <= 1024 else 0
+    R, W = next(((R, W) for R, W in ((2, 1), (4, 1), (8, 1), (4, 4), (8, 4), (16, 4)) if rlen <= 64 * R * W), (0, 0))
     for p in range(P):
         n = pos0 + p + 1
         assert n <= S
         if R:
-            assert n <= 64 * R  # the buffer range check zeroes the rest; stores are masked by n
+            assert n <= 64 * W * R  # the buffer range check zeroes the rest; stores are masked by n
+        if W > 1:  # the serial sum reads the exponentials in pieces of 64
+            inb("pf softmax ex LDS", np.arange(0, n, 64) + 63, 64 * W * R)
         for h in range(nh):
             inb("pf softmax row", (h * P + p) * S + np.arange(n), nh * P * S)
 
 
-def pf_pv_rb(HD, nh, nkv, S, P, pos0, e, PP):
-    """k_pf_pv_rb<HD> over grid (n_heads, ceil(P / (2048/HD))) x 256 threads, with Wo's image."""
-    T, VC = 2048 // HD, PF_VC
-    VR, PR = VC * HD // 4 // WG, T * VC // WG
+def pf_pv_m(HD, nh, nkv, S, P, pos0, e, PP, per_set=True):
+    """k_pf_pv_m<HD> over grid (n_heads * CG/CW, ceil(P / (16*TW))) x 4 waves, with Wo's image. per_set: a
+    set's base is in its resources; else in the scalar offset of loads from the whole array's resource."""
+    NB = 3
+    CG = (HD + 31) // 32
+    CW = 4 if CG % 4 == 0 else 2 if CG % 2 == 0 else 1
+    TW = 4 // CW
     group, kvd = nh // nkv, nkv * HD
-    ng = (P + T - 1) // T
-    q4 = ng // 4
-    gy = np.arange(ng)
-    grp = np.where((ng % 4 == 0) & ((gy // max(q4, 1)) % 2 == 1), (gy // max(q4, 1)) * q4 + (q4 - 1 - gy % max(q4, 1)), gy)
-    assert np.array_equal(np.sort(grp), np.arange(ng)), "every token group once"
-    tid = np.arange(WG)
-    ev = (np.arange(VR)[:, None] * WG + tid[None, :]).ravel()
-    inb("pf pv LDS vs", (ev // (HD // 4)) * HD + 4 * (ev % (HD // 4)) + 3, VC * HD)
-    ep = (np.arange(PR)[:, None] * WG + tid[None, :]).ravel()
-    inb("pf pv LDS ps", (ep % VC) * T + ep // VC, VC * T)
-    tg, cg = tid // (HD // 2), tid % (HD // 2)
-    assert 4 * tg.max() + 3 < T and 2 * cg.max() + 1 < HD
+    G = (P + 16 * TW - 1) // (16 * TW)
+    half, y = (G + 1) // 2, np.arange(G)
+    grp = np.where(y < half, G - 1 - y, y - half)
+    assert np.array_equal(np.sort(grp), np.arange(G)), "every token group once"
+    l = np.arange(64)
+    hi, row0 = l >> 5, 4 * (l >> 4)
     nblk = nh * HD // 32
-    for g in grp:
-        p0 = int(g) * T
-        np_ = min(T, P - p0)
+    inb("pf pv tile LDS", (row0 + 3) * 36 + 16 + (l & 15), 16 * 36)
+    for p0 in range(0, P, 16):
+        np_ = min(16, P - p0)
         tmax = pos0 + p0 + np_
+        # sets loaded: two before the loop, then one per set used, two ahead
+        sets = sorted({8 * w for w in range(NB - 1)} | {t + 8 * (NB - 1) for t in range(0, tmax, 8)})
+        assert sets[-1] + 8 > tmax
         for h in range(nh):
             kvh = h // group
-            for c0 in range(0, tmax, VC):
-                t = ev // (HD // 4)
-                tc = np.minimum(c0 + t, tmax - 1)
-                inb("pf pv V", kvh * HD + tc * kvd + 4 * (ev % (HD // 4)) + 3, e.V)
-                kk, tt = ep // VC, c0 + ep % VC
-                on = (kk < np_) & (tt <= pos0 + p0 + kk)
-                inb("pf pv att", ((h * P + p0 + kk) * S + tt)[on], nh * P * S)
-            for a in range(4):
-                kk = 4 * tg + a
-                on = kk < np_
-                inb("pf pv out", ((p0 + kk) * nh * HD + h * HD + 2 * cg + 1)[on], P * nh * HD)
-                b = h * (HD // 32) + (cg >> 4)
-                assert b.max() < nblk
-                j = cg & 15
-                inb("pf pv image (Q4 order)", ((b * PP + p0 + kk) * 32 + 8 * (j >> 2) + 7)[on & ((j & 3) == 0)], nblk * PP * 32)
-                inb("pf pv image (Q8 order)", ((b * PP + p0 + kk) * 32 + 2 * j + 3)[on & ((j & 1) == 0)], nblk * PP * 32)
-                inb("pf pv image d", (b * PP + p0 + kk)[on & (j == 0)], nblk * PP)
+            pbase, vbase = (h * P + p0) * S, kvh * HD
+            pl = np.where(p0 + (l & 15) < P, l & 15, np_ - 1)
+            for c0 in range(0, 32 * CG, 32):
+                cl = np.where(c0 + (l & 31) < HD, c0 + (l & 31), 0)
+                for t in sets:
+                    po = pl * S + 4 * hi
+                    vo = cl + (4 * hi + np.arange(4)[:, None]) * kvd
+                    if not per_set:
+                        inb("pf pv att", pbase + t + po, nh * P * S)
+                        inb("pf pv V", vbase + t * kvd + vo, e.V)
+                        continue
+                    n = max(0, min(8, S - t))
+                    pn, vn = (np_ * S - t, n * kvd - kvh * HD) if n else (0, 0)
+                    assert 0 <= pn < 1 << 30 and 0 <= vn < 1 << 30
+                    if n:  # the resources lie in their arrays
+                        inb("pf pv att resource", np.array([pbase + t, pbase + t + pn - 1]), nh * P * S)
+                        inb("pf pv V resource", np.array([vbase + t * kvd, vbase + t * kvd + vn - 1]), e.V)
+                    # and hold every value that is used: positions some token of the group sees
+                    for q in range(8):
+                        if t + q < tmax:
+                            on = hi == q // 4
+                            inb("pf pv p used", (po + q % 4)[on], pn)
+                            inb("pf pv v used", vo[q % 4][on], vn)
+                if c0 + 32 <= HD:
+                    kk = np.concatenate([8 * r + (l >> 3) for r in range(2)])
+                    on, b = kk < np_, h * (HD // 32) + c0 // 32
+                    assert b < nblk
+                    inb("pf pv image", ((b * PP + p0 + kk) * 32 + 4 * (np.tile(l, 2) & 7) + 3)[on], nblk * PP * 32)
+                    inb("pf pv image d", (b * PP + p0 + kk)[on], nblk * PP)
+                for b in range(2):
+                    c = c0 + 16 * b + (l & 15)
+                    for el in range(4):
+                        on = (row0 + el < np_) & (c < HD)
+                        inb("pf pv out", (((p0 + row0 + el) * nh + h) * HD + c)[on], P * nh * HD)
 
 
-@pytest.mark.parametrize("HD,nh,nkv,S", [(128, 32, 32, 640), (128, 2, 2, 1300), (64, 12, 12, 1024),
-                                         (64, 32, 4, 2048), (64, 4, 1, 300)])
-@pytest.mark.parametrize("P,pos0", [(1, 0), (5, 0), (64, 0), (65, 3), (130, 200), (512, 0), (300, 700)])
+# (300, 0), (299, 1), (1, 299), (130, 510) and (9, 1015) end at max_seq of some shape
+@pytest.mark.parametrize("HD,nh,nkv,S", [(128, 4, 4, 640), (128, 2, 2, 1300), (64, 3, 3, 1024), (64, 8, 2, 2048),
+                                         (64, 4, 1, 300), (48, 6, 2, 300), (48, 2, 1, 4099)])
+@pytest.mark.parametrize("P,pos0", [(1, 0), (5, 0), (64, 0), (65, 3), (130, 200), (300, 0), (299, 1), (1, 299),
+                                    (130, 510), (9, 1015), (512, 0), (300, 700), (3, 4096)])
 def test_prefill_tile_kernel_indices_in_bounds(HD, nh, nkv, S, P, pos0):
     if pos0 + P > S:
         pytest.skip("the launcher takes pos0 + P <= max_seq only")
@@ -317,14 +341,14 @@ def test_prefill_tile_kernel_indices_in_bounds(HD, nh, nkv, S, P, pos0):
     PP = (min(S, 512) + 127) // 128 * 128  # the model's pf_pp
     if P > PP:
         pytest.skip("a pass holds at most pf_cap tokens")
-    pf_scores_rb(HD, nh, nkv, S, P, pos0, e)
+    pf_scores_m(HD, nh, nkv, S, P, pos0, e)
     pf_softmax(nh, S, P, pos0)
-    pf_pv_rb(HD, nh, nkv, S, P, pos0, e, PP)
+    pf_pv_m(HD, nh, nkv, S, P, pos0, e, PP)
 
 
 def test_prefill_model_catches_an_unclamped_position():
-    """Not vacuous: k_pf_scores_rb's K^T tile reads positions c0 .. c0+63 clamped to max_seq-1; without
-    the clamp the last tile of a context ending at max_seq = 1300 reads past the last kv head's K."""
+    """Not vacuous: k_pf_scores_m reads positions c0 .. c0+63 clamped to max_seq-1; without the clamp the last
+    tile of a context ending at max_seq = 1300 reads past the last kv head's K."""
     HD, nkv, S = 128, 2, 1300
     K = Extents(2, nkv, HD, S).K
     c0 = 1280
@@ -332,3 +356,12 @@ def test_prefill_model_catches_an_unclamped_position():
     inb("kept clamp", ((nkv - 1) * HD + HD - 1) * S + np.minimum(t, S - 1), K)
     with pytest.raises(AssertionError):
         inb("planted", ((nkv - 1) * HD + HD - 1) * S + t, K)
+
+
+@pytest.mark.parametrize("P,pos0", [(1, 0), (1, 299), (300, 0)])
+def test_prefill_model_catches_positions_in_the_scalar_offset(P, pos0):
+    """Not vacuous: with the position in the scalar offset, which the range check need not cover, the sets
+    that P.V loads ahead leave V at the end of a context, and the probabilities of a single token."""
+    e = Extents(4, 1, 64, 300)
+    with pytest.raises(AssertionError):
+        pf_pv_m(64, 4, 1, 300 if pos0 + P > 1 else 8, P, pos0, e, 128 if P == 1 else 512, per_set=False)

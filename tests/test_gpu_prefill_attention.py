@@ -52,7 +52,9 @@ def want(oracle, q, kt, v, P, pos0, n_heads, n_kv, hd, scale):
 @pytest.mark.parametrize("hd,n_heads,n_kv,P,pos0,S", [
     (48, 2, 1, 67, 0, 67), (48, 2, 2, 18, 61, 80), (64, 2, 1, 33, 0, 33), (64, 2, 2, 17, 239, 257),
     (128, 1, 1, 16, 0, 16), (128, 2, 1, 15, 499, 515), (128, 1, 1, 3, 1021, 1027), (64, 1, 1, 5, 2044, 2049),
-    (64, 1, 1, 2, 4095, 4097), (32, 2, 2, 19, 100, 121)])
+    (64, 1, 1, 2, 4095, 4097), (32, 2, 2, 19, 100, 121),
+    # contexts that end at max_seq: the last 4-position loads run past the last row, the sets loaded ahead past V
+    (64, 1, 1, 1, 0, 1), (64, 2, 1, 1, 5, 6), (128, 2, 2, 2, 9, 11), (48, 2, 1, 17, 6, 23), (128, 1, 1, 16, 493, 509)])
 def test_against_restatement(gpu, oracle, hd, n_heads, n_kv, P, pos0, S):
     print("case", hd, n_heads, n_kv, P, pos0, S, flush=True)
     rs = np.random.default_rng(hd + P + pos0)
@@ -62,7 +64,7 @@ def test_against_restatement(gpu, oracle, hd, n_heads, n_kv, P, pos0, S):
     q[0, 0, :4] = [0.0, -0.0, 1e-40, 3e38]  # signed zeros, a subnormal, a product that overflows
     kt[:4, 0] = [-1.0, 1.0, 1e-3, 0.25]
     v[pos0 + P:] = np.nan  # positions nobody sees
-    v[0, 0], v[1, 1] = -0.0, 1e-41
+    v[0, 0], v[min(1, S - 1), 1] = -0.0, 1e-41
     scale = 1.0 / np.sqrt(np.float32(hd))
     got = run(gpu, q, kt, v, P, pos0, n_heads, n_kv, hd, S, scale)
     ref = want(oracle, q, kt, v, P, pos0, n_heads, n_kv, hd, scale)
