@@ -162,8 +162,8 @@ int qmh_launch_pf_quant(const float *x, int ldx, const float *w, float eps, int 
                         int PP, int perm8, void *stream);
 int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream);
 /* causal attention of P tokens at positions pos0.. over the caches; att: scratch [n_heads][P][max_seq].
- * xc != NULL (head_dim 128 or 64 only): out is written as its Q8_0 image instead (xc, xd, PP tokens per
- * block, perm8: the Q4_0 consumers' byte order), as qmh_launch_pf_quant would write it */
+ * xc != NULL (head_dim 128 or 64 only): out's Q8_0 image is written (xc, xd, PP tokens per block, perm8: the
+ * Q4_0 consumers' byte order), as qmh_launch_pf_quant would write it; what out holds is then not defined */
 int qmh_launch_pf_attention(const float *Q, const float *Kt, const float *V, float *att, float *out, int P, int pos0,
                             int n_heads, int n_kv, int hd, int max_seq, float scale, int8_t *xc, float *xd, int PP,
                             int perm8, void *stream);

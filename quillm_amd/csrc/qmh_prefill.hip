@@ -1648,7 +1648,7 @@ extern "C" int qmh_launch_pf_attention(const float *Q, const float *Kt, const fl
                                        int pos0, int n_heads, int n_kv, int hd, int max_seq, float scale, int8_t *xc,
                                        float *xd, int PP, int perm8, void *stream) {
     if (hd > 128 || hd % 4 || pos0 + P > max_seq || P < 1) return (int)hipErrorInvalidValue;
-    // the output's quantized image comes only from k_pf_pv_m (head_dim 128 or 64: whole blocks)
+    // the output's quantized image: from k_pf_pv_m (head_dim 128 or 64: whole blocks), or from out after k_pf_pv
     if (xc && (!xd || (hd != 128 && hd != 64) || P > PP)) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
     const int ng = (P + QMH_PF_TOK - 1) / QMH_PF_TOK, nz = (pos0 + P + QMH_WG - 1) / QMH_WG;
@@ -1657,7 +1657,6 @@ extern "C" int qmh_launch_pf_attention(const float *Q, const float *Kt, const fl
     // head_dim 48, 64, 128: products from MFMAs (16 rows of probabilities and 8 of V within 32-bit offsets,
     // queries read as float4s)
     const bool mf = (hd == 128 || hd == 64 || hd == 48) && max_seq < 1 << 26 && n_kv < 1 << 16 && ((uintptr_t)Q & 15) == 0;
-    if (xc && !mf) return (int)hipErrorInvalidValue;
 #define PF_HD(K_, G_, ...)                                                         \
     do {                                                                           \
         if (hd == 128) hipLaunchKernelGGL(K_<128>, G_, wg, 0, s, __VA_ARGS__);     \
@@ -1687,5 +1686,7 @@ extern "C" int qmh_launch_pf_attention(const float *Q, const float *Kt, const fl
     else
         hipLaunchKernelGGL(k_pf_pv, dim3(n_heads, ng), wg, 0, s, att, V, out, P, pos0, n_heads, n_kv, hd, max_seq);
 #undef PF_HD
-    return (int)hipGetLastError();
+    const int rc = (int)hipGetLastError();
+    if (rc || !xc || mf) return rc;
+    return qmh_launch_pf_quant(out, n_heads * hd, nullptr, 0.0f, n_heads * hd, P, xc, xd, PP, perm8, stream);
 }

@@ -12,23 +12,33 @@ from _boundary import softmax_boundary_input
 pytestmark = pytest.mark.gpu
 
 
-def run(gpu, q, kt, v, P, pos0, n_heads, n_kv, hd, S, scale):
+def run(gpu, q, kt, v, P, pos0, n_heads, n_kv, hd, S, scale, image=None, skew=0):
+    """out, or with image (perm8: 0 or 1) its quantized codes and scales; the queries skew bytes past alignment, kt and
+    v arrays or device buffers"""
     L = gpu.load_library()
     fn = L.qmh_launch_pf_attention
     fn.restype = ctypes.c_int
     vp, i32 = ctypes.c_void_p, ctypes.c_int
     fn.argtypes = [vp] * 5 + [i32] * 6 + [ctypes.c_float, vp, vp, i32, i32, vp]
-    b = [gpu.DeviceBuffer.from_array(a) for a in (q, kt, v)]
+    b = [gpu.DeviceBuffer(q.nbytes + skew)] + [gpu.DeviceBuffer.from_array(a) for a in (kt, v) if isinstance(a, np.ndarray)]
+    dk, dv = b[1:] or (kt, v)
     att, out = gpu.DeviceBuffer(n_heads * P * S * 4), gpu.DeviceBuffer(P * n_heads * hd * 4)
+    PP = 128
+    xc, xd = gpu.DeviceBuffer(PP * n_heads * hd), gpu.DeviceBuffer(PP * n_heads * hd // 32 * 4)
     try:
-        assert gpu.load_library().qmh_memset(att.ptr, 0xff, att.nbytes) == 0  # NaN wherever nothing is written
-        rc = fn(b[0].ptr, b[1].ptr, b[2].ptr, att.ptr, out.ptr, P, pos0, n_heads, n_kv, hd, S, float(scale), None, None,
-                128, 0, L.qmh_stream())
+        assert L.qmh_memcpy_h2d(b[0].ptr + skew, q.ctypes.data, q.nbytes) == 0
+        for x in (att, out, xc, xd):
+            assert L.qmh_memset(x.ptr, 0xff, x.nbytes) == 0  # NaN wherever nothing is written
+        rc = fn(b[0].ptr + skew, dk.ptr, dv.ptr, att.ptr, out.ptr, P, pos0, n_heads, n_kv, hd, S, float(scale),
+                None if image is None else xc.ptr, None if image is None else xd.ptr, PP, image or 0, L.qmh_stream())
         assert rc == 0
         gpu.sync()
-        return out.to_array(np.float32).reshape(P, n_heads, hd)
+        if image is None:
+            return out.to_array(np.float32).reshape(P, n_heads, hd)
+        codes = xc.to_array(np.int8).reshape(-1, PP, 32)[:, :P]
+        return codes, xd.to_array(np.float32).reshape(-1, PP)[:, :P]
     finally:
-        for x in b + [att, out]:
+        for x in b + [att, out, xc, xd]:
             x.free()
 
 
@@ -61,7 +71,7 @@ def test_against_restatement(gpu, oracle, hd, n_heads, n_kv, P, pos0, S):
     q = rs.standard_normal((P, n_heads, hd)).astype(np.float32)
     kt = rs.standard_normal((n_kv * hd, S)).astype(np.float32)
     v = rs.standard_normal((S, n_kv * hd)).astype(np.float32)
-    q[0, 0, :4] = [0.0, -0.0, 1e-40, 3e38]  # signed zeros, a subnormal, a product that overflows
+    q[0, 0, :4] = [0.0, -0.0, 1e-40, 3e38]  # signed zeros, a subnormal, products that overflow
     kt[:4, 0] = [-1.0, 1.0, 1e-3, 0.25]
     v[pos0 + P:] = np.nan  # positions nobody sees
     v[0, 0], v[min(1, S - 1), 1] = -0.0, 1e-41
@@ -88,3 +98,57 @@ def test_serial_sum(gpu, oracle, n):
         v[idx, np.arange(hd)] = 1.0
         got = run(gpu, q, kt, v, 1, n - 1, 1, 1, hd, n, 1.0)
         assert np.array_equal(got[0, 0].view(np.uint32), oracle.softmax(s)[idx].view(np.uint32)), (n, seed)
+
+
+# the quantized image from the general kernels, where the queries' alignment keeps the others out: the same
+# codes and scales, both byte orders
+@pytest.mark.parametrize("hd,n_heads,n_kv,P,pos0,S", [(64, 2, 1, 19, 3, 64), (128, 2, 2, 5, 300, 310)])
+@pytest.mark.parametrize("perm8", [0, 1])
+def test_image_of_unaligned_queries(gpu, hd, n_heads, n_kv, P, pos0, S, perm8):
+    print("case", hd, n_heads, n_kv, P, pos0, S, perm8, flush=True)
+    rs = np.random.default_rng(hd + P)
+    q = rs.standard_normal((P, n_heads, hd)).astype(np.float32)
+    kt = rs.standard_normal((n_kv * hd, S)).astype(np.float32)
+    v = rs.standard_normal((S, n_kv * hd)).astype(np.float32)
+    a = run(gpu, q, kt, v, P, pos0, n_heads, n_kv, hd, S, hd ** -0.5, image=perm8)
+    b = run(gpu, q, kt, v, P, pos0, n_heads, n_kv, hd, S, hd ** -0.5, image=perm8, skew=4)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1].view(np.uint32), b[1].view(np.uint32))
+
+
+# a layer's keys and values past 4 GiB: 64 heads x 64 dimensions, a token at the end of 262208 positions, random
+# values in the first and last heads' keys and in the first and last 64 positions' V (zeros elsewhere), the
+# probabilities of every position. Then the same token's image, from both sets of kernels.
+def test_caches_past_4_gib(gpu, oracle):
+    print("case 4 GiB", flush=True)
+    nh, hd, S, n = 64, 64, 262208, 64
+    L = gpu.load_library()
+    rs = np.random.default_rng(9)
+    q = rs.standard_normal((1, nh, hd)).astype(np.float32)
+    k = {h: 0.1 * rs.standard_normal((hd, S)).astype(np.float32) for h in (0, nh - 1)}
+    v = {t: rs.standard_normal((n, nh * hd)).astype(np.float32) for t in (0, S - n)}
+    dk, dv = gpu.DeviceBuffer(4 * nh * hd * S), gpu.DeviceBuffer(4 * nh * hd * S)
+    try:
+        for d in (dk, dv):
+            assert L.qmh_memset(d.ptr, 0, d.nbytes) == 0
+        for h, x in k.items():
+            assert L.qmh_memcpy_h2d(dk.ptr + 4 * h * hd * S, x.ctypes.data, x.nbytes) == 0
+        for t, x in v.items():
+            assert L.qmh_memcpy_h2d(dv.ptr + 4 * t * nh * hd, x.ctypes.data, x.nbytes) == 0
+        scale = np.float32(hd ** -0.5)
+        got = run(gpu, q, dk, dv, 1, S - 1, nh, nh, hd, S, scale)
+        images = [run(gpu, q, dk, dv, 1, S - 1, nh, nh, hd, S, scale, image=1, skew=s) for s in (0, 4)]
+    finally:
+        dk.free()
+        dv.free()
+    for h in k:
+        s = np.zeros(S, np.float32)
+        for d in range(hd):
+            s = s + q[0, h, d] * k[h][d]
+        pr = oracle.softmax(s * scale)
+        acc = np.zeros(hd, np.float32)  # zeros of V add +0 to a chain from +0
+        for t0, x in v.items():
+            for t in range(n):
+                acc = acc + pr[t0 + t] * x[t, h * hd:(h + 1) * hd]
+        assert np.array_equal(got[0, h].view(np.uint32), acc.view(np.uint32)), h
+    assert np.array_equal(images[0][0], images[1][0])
+    assert np.array_equal(images[0][1].view(np.uint32), images[1][1].view(np.uint32))
