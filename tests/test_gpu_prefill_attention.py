@@ -81,6 +81,26 @@ def test_against_restatement(gpu, oracle, hd, n_heads, n_kv, P, pos0, S):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), np.argwhere(got.view(np.uint32) != ref.view(np.uint32))[:5]
 
 
+# scores and P.V whose products and sums are all subnormal: score chains below 2^-126, which the scale brings to the
+# order of one, and values of V below 2^-126. A product or a sum flushed to zero would change every output.
+@pytest.mark.parametrize("hd,n_heads,n_kv,P,pos0", [(48, 2, 1, 18, 0), (64, 2, 2, 33, 70), (128, 2, 1, 17, 130)])
+def test_subnormal_chains(gpu, oracle, hd, n_heads, n_kv, P, pos0):
+    print("case", hd, n_heads, n_kv, P, pos0, flush=True)
+    rs = np.random.default_rng(hd)
+    S = pos0 + P
+    q = (rs.standard_normal((P, n_heads, hd)) * 2.0 ** -66).astype(np.float32)
+    kt = (rs.standard_normal((n_kv * hd, S)) * 2.0 ** -66).astype(np.float32)
+    v = (rs.standard_normal((S, n_kv * hd)) * 2.0 ** -129).astype(np.float32)
+    scale = np.float32(2.0 ** 127)
+    chains = np.einsum("phd,hdt->pht", q.astype(np.float64), np.stack([kt[h // (n_heads // n_kv) * hd:][:hd]
+                                                                       for h in range(n_heads)]).astype(np.float64))
+    assert np.abs(chains).max() < 2.0 ** -126 and np.abs(chains * float(scale)).max() > 0.1
+    ref = want(oracle, q, kt, v, P, pos0, n_heads, n_kv, hd, scale)
+    assert 0 < np.abs(ref).max() < 2.0 ** -126
+    got = run(gpu, q, kt, v, P, pos0, n_heads, n_kv, hd, S, scale)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
 # rows whose sum of exponentials sits on a float midpoint of its reciprocal: the tree sum cannot decide it,
 # and the reference's serial sum is taken. Scores are given exactly (query 1, 0, 0, ..; key row 0 the score).
 @pytest.mark.parametrize("n", [90, 200, 300, 500, 700, 1500, 3000])
