@@ -108,16 +108,23 @@ int qmh_launch_attn_batch(const float *Q, const float *Kt, const float *V, long 
 enum { QMH_PF_STORE = 0, QMH_PF_ADD = 1, QMH_PF_QKV = 2, QMH_PF_SWIGLU = 3 };
 /* which matmul runs P tokens: the skinny one (a 16-row group per workgroup, one workgroup per CU, every weight
  * streamed once) or the tiled one. The skinny matmul's time grows with the terms, rows * P; the tiled one's is the
- * length of its chains until the tiles fill the chip (both grow alike with the columns). Timed, us, skinny -> tiled:
- * 32000 rows x 4096 columns 39 -> 32 at 8 tokens, 61 -> 33 at 16; 2 x 11008 (W1 | W3) x 4096 34 -> 36 at 8, 45 -> 36 at
- * 16, 130 -> 40 at 64; 12288 x 4096 26 -> 32 at 16, 39 -> 32 at 32; 2 x 5632 x 2048 18 -> 19 at 16, 25 -> 19 at 32; 4096
- * rows stay ahead in the skinny one up to 64 tokens (59 -> 63). Below 8 tokens only the skinny one (and the
- * multi-token matvec) is used, past QMH_PF_SKINNY_P only the tiled one. */
+ * length of its chains until the tiles fill the chip. Both grow alike with the columns, down to about 512. Timed,
+ * us, skinny -> tiled: 32000 rows x 4096 columns 39 -> 32 at 8 tokens, 61 -> 33 at 16; 2 x 11008 (W1 | W3) x 4096 34 -> 36
+ * at 8, 45 -> 36 at 16, 130 -> 40 at 64; 12288 x 4096 26 -> 32 at 16, 39 -> 32 at 32; 2 x 5632 x 2048 18 -> 19 at 16, 25 -> 19
+ * at 32; 4096 rows stay ahead in the skinny one up to 64 tokens (59 -> 63); 32000 x 768 19 -> 11 at 33; 32000 x 288
+ * 13 -> 7 at 10, 17.5 -> 9.5 at 64.
+ * Below 16 blocks of columns what the tiled one spends outside its chains, most of all from 33 tokens on, where its
+ * workgroups hold two token tiles, moves the line: at 64 tokens, 4704 rows x 64 columns 3.5 -> 4.7, 9376 4.2 -> 5.7, 32000
+ * 8.6 -> 7.0; 6576 x 256 5.2 -> 6.5, 9376 6.2 -> 6.3, 14064 7.7 -> 6.8; W1 | W3 with W2's input image 2 x 2352 x 64 7.1 -> 8.4,
+ * 2 x 4688 8.7 -> 8.5, 2 x 2352 x 384 9.9 -> 10.1, 2 x 4688 16 -> 10. Up to 32 tokens it does not (9376 x 128 6.4 -> 5.7 at
+ * 32; at 64 columns 5.1 -> 5.5).
+ * Below 8 tokens only the skinny one (and the multi-token matvec) is used, past QMH_PF_SKINNY_P only the tiled one. */
 #ifndef QMH_PF_SKINNY_P
 #define QMH_PF_SKINNY_P 64
 #endif
-static inline int qmh_pf_tiled(int P, int rows, int il) {
-    return P > QMH_PF_SKINNY_P || (P >= 8 && (long long)P * rows * (il ? 2 : 1) >= 300000);
+static inline int qmh_pf_tiled(int P, int rows, int nb, int il) {
+    const int from = P <= 32 || nb >= 16 ? 300000 : il ? 400000 : nb >= 8 ? 450000 : 1000000;
+    return P > QMH_PF_SKINNY_P || (P >= 8 && (long long)P * rows * (il ? 2 : 1) >= from);
 }
 typedef struct {
     /* weight: tiled codes/scales as for the matvec; il: interleaved W1 | W3 tiles */

@@ -1068,7 +1068,7 @@ extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
     if ((a->epi == QMH_PF_SWIGLU) != (a->il != 0)) return (int)hipErrorInvalidValue;
     if (a->dtype != QMH_Q4 && a->dtype != QMH_Q8) return (int)hipErrorInvalidValue;
     // the image output exists only in the tiled matmul's SwiGLU epilogue
-    if (a->qxc && (a->epi != QMH_PF_SWIGLU || !a->qxd || !qmh_pf_tiled(a->P, a->rows, a->il))) return (int)hipErrorInvalidValue;
+    if (a->qxc && (a->epi != QMH_PF_SWIGLU || !a->qxd || !qmh_pf_tiled(a->P, a->rows, a->nb, a->il))) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
     if (a->xf && (a->nxf < 1 || a->nxf > 32 * a->nb || a->ldxf < a->nxf)) return (int)hipErrorInvalidValue;
     // the multi-token matvec when one tile's terms fit its LDS with the records. It quantizes a plain
@@ -1115,7 +1115,7 @@ extern "C" int qmh_launch_pf_gemm(const qmh_pf_args *a, void *stream) {
 #undef BMV_GO
         return (int)hipGetLastError();
     }
-    if (!qmh_pf_tiled(a->P, a->rows, a->il)) {  // decode-sized batches: the skinny matmul streams every weight once
+    if (!qmh_pf_tiled(a->P, a->rows, a->nb, a->il)) {  // decode-sized batches: the skinny matmul streams every weight once
         const dim3 g((a->rows + 15) / 16);
         const int nm = a->il ? 2 : 1;
         const size_t lds = (size_t)sk_round(a->nb, nm, a->P) * nm * 16 * a->P * sizeof(float);

@@ -1131,7 +1131,7 @@ static int pf_layer(qmh_model *m, int l, int P, int pos, const pf_seqs *bt, hipS
     a.out0 = m->d_pf_hb;
     a.ld0 = H;
     /* from the tiled matmul hb is written only as W2's quantized image */
-    const int hb_image = qmh_pf_tiled(P, H, 1);
+    const int hb_image = qmh_pf_tiled(P, H, L->w13.nb, 1);
     if (hb_image) {
         a.qxc = m->d_pf_xc2;
         a.qxd = m->d_pf_xd2;

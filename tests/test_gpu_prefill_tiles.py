@@ -101,9 +101,9 @@ def test_nonfinite_scales(gpu, monkeypatch, where, vocab, wt):
         check(m, monkeypatch, 70, vocab)
 
 
-# both sides of the rule that takes 8 to 64 tokens to the tiled matmul (300000 rows x tokens), for the output
-# (row counts that end inside tiles) and for W1 | W3, whose input image to W2 changes with it; one and two
-# token tiles
+# both sides of the rule that takes 8 to 64 tokens to the tiled matmul (300000 rows x tokens up to 32 tokens), for
+# the output (row counts that end inside tiles) and for W1 | W3, whose input image to W2 changes with it; one and
+# two token tiles
 @pytest.mark.parametrize("wt", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("hidden,vocab,P", [(200, 37501, 7), (200, 37500, 8), (200, 37499, 8), (200, 9376, 32),
                                             (200, 9376, 31), (200, 9091, 33), (4688, 300, 32), (4687, 300, 32),
@@ -111,4 +111,16 @@ def test_nonfinite_scales(gpu, monkeypatch, where, vocab, wt):
 def test_few_token_rule(gpu, monkeypatch, hidden, vocab, P, wt):
     print(f"case {hidden} {vocab} {P} {wt}", flush=True)
     with model(gpu, 72, hidden, 6, 2, vocab, 128, wt) as m:
+        check(m, monkeypatch, P, vocab)
+
+
+# the same from 33 tokens on, where the line depends on the columns: below 8 blocks (1000000; W1 | W3 400000), below
+# 16 (450000), from 16 on (300000)
+@pytest.mark.parametrize("dim,hidden,vocab,P", [(72, 200, 15625, 64), (72, 200, 15624, 64), (72, 3125, 300, 64),
+                                                (72, 3124, 300, 64), (288, 32, 7032, 64), (288, 32, 7031, 64),
+                                                (288, 6061, 300, 33), (288, 6060, 300, 33), (528, 32, 4688, 64),
+                                                (528, 32, 4687, 64)])
+def test_few_token_rule_by_columns(gpu, monkeypatch, dim, hidden, vocab, P):
+    print(f"case {dim} {hidden} {vocab} {P}", flush=True)
+    with model(gpu, dim, hidden, 6, 2, vocab, 128, "q4_0") as m:
         check(m, monkeypatch, P, vocab)
