@@ -1257,14 +1257,15 @@ __global__ __launch_bounds__(QMH_WG, 4) void k_pf_scores_m(const float *__restri
         __builtin_amdgcn_wave_barrier();
         q = qs[wave][l & 15];
     }
-    const float *kt = Kt + (size_t)kvh * HD * max_seq;  // a uniform row pointer per dimension, the lane's position clamped
+    // every offset below lies in the kv head's keys: positions clamped to max_seq - 1, dimensions below HD
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(Kt + (size_t)kvh * HD * max_seq), (short)0, (int)((uint32_t)HD * (uint32_t)max_seq * 4u), 0x00020000);
     pf_v4f qv[2][DG / 4];
     float kv[2][DG];
     auto load = [&](int d0, int w) {
 #pragma unroll
         for (int d = 0; d < DG / 4; d++) qv[w][d] = *(const pf_v4f *)(q + d0 + 4 * d);
 #pragma unroll
-        for (int d = 0; d < DG; d++) kv[w][d] = (kt + (size_t)(d0 + d) * max_seq)[(uint32_t)tc];
+        for (int d = 0; d < DG; d++) kv[w][d] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, tc * 4, (uint32_t)(d0 + d) * (uint32_t)max_seq * 4u, 0));
     };
     float s[16];
     pf_v16f z;
@@ -1560,29 +1561,28 @@ __global__ __launch_bounds__(QMH_WG, 4) void k_pf_pv_m(const float *__restrict__
     const int np = min(16, P - p0), kvh = h / (n_heads / n_kv), kvd = HD * n_kv;
     const int tall = pos0 + p0 + 1, tmax = pos0 + p0 + np;  // positions seen by every token, by some token
     const int pl = p0 + (l & 15), cl = c0 + (l & 31);
-    // Resources of one set of 8 positions, t .. t + 7: the token group's probabilities from position t of its
-    // first row to the end of its last one, V from position t's row to the eighth's, or to the last of
-    // max_seq. The sets loaded ahead run past the last position, and a 4-position load past the last row's
-    // end: a range check on the lane's offset alone reads those as 0, and they are not used. So each set has
-    // its base in its resources (scalar arithmetic) and nothing in the scalar offset, which the check need not
-    // cover.
-    const float *pbase = att + ((size_t)h * P + p0) * max_seq, *vbase = V + (size_t)kvh * HD;
-    const uint32_t po = ((uint32_t)(pl < P ? l & 15 : np - 1) * (uint32_t)max_seq + 4u * hi) * 4u;
-    uint32_t vo[4];
+    // Resources: the token group's probabilities, and per j the kv head's V from row j. The sets loaded ahead
+    // run past the last position, and a 4-position load past the last row's end: the range check reads those
+    // as 0, and they are not used. It need cover the lane's offset only, so the position is in there and nothing
+    // in the scalar offset.
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(att + ((size_t)h * P + p0) * max_seq), (short)0, (int)((uint32_t)np * (uint32_t)max_seq * 4u), 0x00020000);
+    __amdgpu_buffer_rsrc_t rv[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) vo[j] = ((uint32_t)(cl < HD ? cl : 0) + (4u * hi + j) * (uint32_t)kvd) * 4u;
+    for (int j = 0; j < 4; j++) {
+        const uint32_t n = j < max_seq ? ((uint32_t)(max_seq - j) * (uint32_t)kvd - (uint32_t)(kvh * HD)) * 4u : 0u;
+        rv[j] = __builtin_amdgcn_make_buffer_rsrc((void *)(V + (size_t)kvh * HD + (size_t)j * kvd), (short)0, (int)n, 0x00020000);
+    }
+    uint32_t po = ((uint32_t)(pl < P ? l & 15 : np - 1) * (uint32_t)max_seq + 4u * hi) * 4u;
+    uint32_t vo = ((uint32_t)(cl < HD ? cl : 0) + 4u * hi * (uint32_t)kvd) * 4u;
+    const uint32_t vst = 32u * (uint32_t)kvd;
     constexpr int NB = 3;  // sets of 8 positions: one used, two in flight
     pf_v4u pr[NB];
     float vr[NB][4];
-    auto load = [&](int t, int w) {
-        const int n = t < max_seq ? (max_seq - t < 8 ? max_seq - t : 8) : 0;  // positions from t on, up to 8
-        const uint32_t pn = n ? ((uint32_t)np * (uint32_t)max_seq - (uint32_t)t) * 4u : 0u;
-        const uint32_t vn = n ? ((uint32_t)n * (uint32_t)kvd - (uint32_t)(kvh * HD)) * 4u : 0u;
-        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)(pbase + t), (short)0, (int)pn, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vbase + (size_t)t * kvd), (short)0, (int)vn, 0x00020000);
+    auto load = [&](int w) {  // the next set
         pr[w] = __builtin_amdgcn_raw_buffer_load_b128(rp, po, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; j++) vr[w][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, vo[j], 0, 0));
+        for (int j = 0; j < 4; j++) vr[w][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv[j], vo, 0, 0));
+        po += 32u, vo += vst;
     };
     float s[8];  // element 4*b + e: token row0 + e, column 16*b + l%16
     pf_v16f z;
@@ -1607,14 +1607,14 @@ __global__ __launch_bounds__(QMH_WG, 4) void k_pf_pv_m(const float *__restrict__
         }
     };
 #pragma unroll
-    for (int w = 0; w < NB - 1; w++) load(8 * w, w);
+    for (int w = 0; w < NB - 1; w++) load(w);
 #pragma unroll 1
     for (int t = 0; t < tmax; t += 8 * NB) {
 #pragma unroll
         for (int w = 0; w < NB; w++) {
             const int tw = t + 8 * w;
             if (tw < tmax) {  // uniform
-                load(tw + 8 * (NB - 1), (w + NB - 1) % NB);
+                load((w + NB - 1) % NB);
                 if (tw + 8 <= tall) group(w, tw, false);
                 else group(w, tw, true);
             }
@@ -1654,9 +1654,10 @@ extern "C" int qmh_launch_pf_attention(const float *Q, const float *Kt, const fl
     const int ng = (P + QMH_PF_TOK - 1) / QMH_PF_TOK, nz = (pos0 + P + QMH_WG - 1) / QMH_WG;
     const int rlen = pos0 + P;  // the longest row
     const dim3 wg(QMH_WG);
-    // head_dim 48, 64, 128: products from MFMAs (16 rows of probabilities and 8 of V within 32-bit offsets,
-    // queries read as float4s)
-    const bool mf = (hd == 128 || hd == 64 || hd == 48) && max_seq < 1 << 26 && n_kv < 1 << 16 && ((uintptr_t)Q & 15) == 0;
+    // head_dim 48, 64, 128: products from MFMAs (a layer's V, with the sets loaded past it, within 32-bit
+    // offsets; queries read as float4s)
+    const bool mf = (hd == 128 || hd == 64 || hd == 48) && (uint64_t)(max_seq + 64ull) * hd * n_kv * 4 < 1ull << 32 &&
+                    ((uintptr_t)Q & 15) == 0;
 #define PF_HD(K_, G_, ...)                                                         \
     do {                                                                           \
         if (hd == 128) hipLaunchKernelGGL(K_<128>, G_, wg, 0, s, __VA_ARGS__);     \

@@ -16,11 +16,10 @@ positions, and checked against its buffer's extent:
   * qmh_launch_pf_attention  quillm_amd/csrc/qmh_prefill.hip, with k_pf_scores_m<HD> (16 x 64 tiles, queries
                              in LDS below 128 dimensions, positions clamped to max_seq - 1),
                              k_pf_softmax_r<R, W> (W waves per row, the exponentials in LDS for W > 1) and
-                             k_pf_pv_m<HD> (sets of 8 positions loaded two ahead, each with buffer
-                             resources of its own, the reversed second half of the token groups and Wo's
-                             quantized image). A buffer load is in bounds when its resource lies in the
-                             array and nothing but the lane's offset, which the range check covers, is
-                             added to the resource's base
+                             k_pf_pv_m<HD> (sets of 8 positions loaded two ahead, the reversed second half
+                             of the token groups and Wo's quantized image). A buffer load that runs past
+                             what is used is in bounds when its resource lies in the array and nothing but
+                             the lane's offset, which the range check covers, is added to its base
 The batched caches are [n_layers][B][kvd * max_seq] (qmh_batch_create, kv_stride = kvd*max_seq,
 quillm_amd/host/qmh_host.c:1337): a sequence's index past its own stride would read the next
 sequence's cache (or, for the last one, past the allocation), so the checks hold each sequence
@@ -269,9 +268,9 @@ def pf_softmax(nh, S, P, pos0):
             inb("pf softmax row", (h * P + p) * S + np.arange(n), nh * P * S)
 
 
-def pf_pv_m(HD, nh, nkv, S, P, pos0, e, PP, per_set=True):
-    """k_pf_pv_m<HD> over grid (n_heads * CG/CW, ceil(P / (16*TW))) x 4 waves, with Wo's image. per_set: a
-    set's base is in its resources; else in the scalar offset of loads from the whole array's resource."""
+def pf_pv_m(HD, nh, nkv, S, P, pos0, e, PP, in_lane=True):
+    """k_pf_pv_m<HD> over grid (n_heads * CG/CW, ceil(P / (16*TW))) x 4 waves, with Wo's image. in_lane: the
+    position is in the lane's offset; else in the scalar offset, which must lie in the arrays by itself."""
     NB = 3
     CG = (HD + 31) // 32
     CW = 4 if CG % 4 == 0 else 2 if CG % 2 == 0 else 1
@@ -298,24 +297,25 @@ def pf_pv_m(HD, nh, nkv, S, P, pos0, e, PP, per_set=True):
             for c0 in range(0, 32 * CG, 32):
                 cl = np.where(c0 + (l & 31) < HD, c0 + (l & 31), 0)
                 for t in sets:
-                    po = pl * S + 4 * hi
-                    vo = cl + (4 * hi + np.arange(4)[:, None]) * kvd
-                    if not per_set:
-                        inb("pf pv att", pbase + t + po, nh * P * S)
-                        inb("pf pv V", vbase + t * kvd + vo, e.V)
+                    po = pl * S + 4 * hi + t
+                    vo = cl + (4 * hi + t) * kvd
+                    rows = np.maximum(S - np.arange(4), 0)  # V from row j on
+                    vn = np.where(rows > 0, rows * kvd - kvh * HD, 0)
+                    if not in_lane:
+                        inb("pf pv att", pbase + po, nh * P * S)
+                        inb("pf pv V", vbase + vo + np.arange(4)[:, None] * kvd, e.V)
                         continue
-                    n = max(0, min(8, S - t))
-                    pn, vn = (np_ * S - t, n * kvd - kvh * HD) if n else (0, 0)
-                    assert 0 <= pn < 1 << 30 and 0 <= vn < 1 << 30
-                    if n:  # the resources lie in their arrays
-                        inb("pf pv att resource", np.array([pbase + t, pbase + t + pn - 1]), nh * P * S)
-                        inb("pf pv V resource", np.array([vbase + t * kvd, vbase + t * kvd + vn - 1]), e.V)
+                    assert 4 * (int(po.max()) + 3) < 1 << 32 and 4 * int(vo.max()) < 1 << 32
+                    # the resources lie in their arrays
+                    inb("pf pv att resource", np.array([pbase, pbase + np_ * S - 1]), nh * P * S)
+                    on = rows > 0
+                    inb("pf pv V resource", (vbase + np.arange(4) * kvd + vn - 1)[on], e.V)
                     # and hold every value that is used: positions some token of the group sees
                     for q in range(8):
                         if t + q < tmax:
                             on = hi == q // 4
-                            inb("pf pv p used", (po + q % 4)[on], pn)
-                            inb("pf pv v used", vo[q % 4][on], vn)
+                            inb("pf pv p used", (po + q % 4)[on], np_ * S)
+                            inb("pf pv v used", vo[on], vn[q % 4])
                 if c0 + 32 <= HD:
                     kk = np.concatenate([8 * r + (l >> 3) for r in range(2)])
                     on, b = kk < np_, h * (HD // 32) + c0 // 32
@@ -364,4 +364,4 @@ def test_prefill_model_catches_positions_in_the_scalar_offset(P, pos0):
     that P.V loads ahead leave V at the end of a context, and the probabilities of a single token."""
     e = Extents(4, 1, 64, 300)
     with pytest.raises(AssertionError):
-        pf_pv_m(64, 4, 1, 300 if pos0 + P > 1 else 8, P, pos0, e, 128 if P == 1 else 512, per_set=False)
+        pf_pv_m(64, 4, 1, 300 if pos0 + P > 1 else 8, P, pos0, e, 128 if P == 1 else 512, in_lane=False)

@@ -135,12 +135,14 @@ def test_image_of_unaligned_queries(gpu, hd, n_heads, n_kv, P, pos0, S, perm8):
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1].view(np.uint32), b[1].view(np.uint32))
 
 
-# a layer's keys and values past 4 GiB: 64 heads x 64 dimensions, a token at the end of 262208 positions, random
-# values in the first and last heads' keys and in the first and last 64 positions' V (zeros elsewhere), the
-# probabilities of every position. Then the same token's image, from both sets of kernels.
-def test_caches_past_4_gib(gpu, oracle):
-    print("case 4 GiB", flush=True)
-    nh, hd, S, n = 64, 64, 262208, 64
+# a layer's keys and values past 2 GiB (the MFMA kernels' 32-bit offsets) and past 4 GiB (the general kernels): 64
+# heads x 64 dimensions, a token at the end of S positions, random values in the first and last heads' keys and in
+# the first and last 64 positions' V (zeros elsewhere), the probabilities of every position. Then the same token's
+# image, from aligned and unaligned queries.
+@pytest.mark.parametrize("S", [262000, 262208])
+def test_large_caches(gpu, oracle, S):
+    print("case", S, flush=True)
+    nh, hd, n = 64, 64, 64
     L = gpu.load_library()
     rs = np.random.default_rng(9)
     q = rs.standard_normal((1, nh, hd)).astype(np.float32)
