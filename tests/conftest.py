@@ -12,6 +12,21 @@ import _bind  # noqa: E402
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a gfx950 (MI355X) device; run with -m gpu")
+    config.addinivalue_line("markers", "compiled_reference: runs the compiled reference's programs")
+
+
+REF_ABSENT = os.path.join(ROOT, "oracle", "_build", "reference_absent")  # written by build() without the sources
+
+
+def pytest_collection_modifyitems(items):
+    """Tests that run the compiled reference are skipped where build() found no reference to compile and none
+    was built before; with its sources there, a missing build stays a failure."""
+    if not os.path.exists(REF_ABSENT) or os.path.exists(_bind.REF_SO):
+        return
+    skip = pytest.mark.skip(reason="the reference's sources were not there to compile")
+    for item in items:
+        if {"ref", "c2_model"} & set(getattr(item, "fixturenames", ())) or item.get_closest_marker("compiled_reference"):
+            item.add_marker(skip)
 
 
 def _need(path, what):

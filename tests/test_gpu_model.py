@@ -104,6 +104,7 @@ def test_max_seq_cap(gpu, small_models):
         assert m.forward(1, 15) is not None and m.forward(1, 16) is None
 
 
+@pytest.mark.compiled_reference
 @pytest.mark.parametrize("name", ["c1", "c2"])
 def test_baseline_config_vs_reference(gpu, tmp_path, name):
     """BASELINE configs c1/c2 (stories15M shape): every position's logits bit-exact with the
@@ -343,6 +344,7 @@ def test_wide_hidden_matches_oracle(gpu, oracle, tmp_path, dim, hidden, heads, k
                         assert np.array_equal(bits(out[i]), bits(wl[i][pos[i]])), f"B={B} step {k} sequence {i}"
 
 
+@pytest.mark.compiled_reference
 @pytest.mark.parametrize("name,dim,hidden,layers,heads,kv,vocab,theta", [
     ("llama3_8b", 4096, 14336, 32, 32, 8, 128256, 500000.0), ("llama2_13b", 5120, 13824, 40, 40, 40, 32000, 10000.0)])
 def test_full_size_shapes_vs_reference(gpu, tmp_path, name, dim, hidden, layers, heads, kv, vocab, theta):

@@ -12,6 +12,7 @@ from _bind import F32, Q4_0, Q8_0, REF_CLI, ref_run, row_bytes
 DT = {"f32": F32, "q8_0": Q8_0, "q4_0": Q4_0}
 
 
+@pytest.mark.compiled_reference
 @pytest.mark.parametrize("shape", ["small", "odd", "mha", "gqa"])
 @pytest.mark.parametrize("wt", ["f32", "q8_0", "q4_0"])
 def test_oracle_forward_bitexact_vs_reference(oracle, small_models, qmh, shape, wt):
@@ -37,6 +38,7 @@ def test_oracle_rejects_bad_token_and_pos(oracle, small_models):
     del ctypes
 
 
+@pytest.mark.compiled_reference
 def test_oracle_c1_shape_bitexact(oracle, qmh, tmp_path):
     """BASELINE config c1 (stories15M shape, Q8_0): a few positions, bit-exact with the reference."""
     w = qmh.WORKLOADS["c1"]
@@ -51,6 +53,7 @@ def test_oracle_c1_shape_bitexact(oracle, qmh, tmp_path):
 
 # ---------------------------------------------------------------------------- generator
 
+@pytest.mark.compiled_reference
 def test_generator_file_is_read_by_reference(small_models):
     path = small_models[("odd", "q4_0")]
     r = subprocess.run([REF_CLI, "info", path], capture_output=True, text=True, timeout=60)
