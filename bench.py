@@ -33,7 +33,9 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0      # MI355X published HBM3E bandwidth
 INT8_PEAK_TOPS = 5000.0    # MI355X dense int8 MFMA
 FP32_MFMA_PEAK_TFS = 157.3  # MI355X dense fp32 MFMA
-VALU_LANE_OPS = 256 * 4 * 16 * 2.4e9  # fp32 VALU lane operations per second (256 CUs x 4 SIMD x 16 lanes x 2.4 GHz)
+# fp32 VALU lane operations per second: 256 CUs x 4 SIMDs, a 64-lane instruction every 2 cycles (measured 2.06 from two
+# or more waves), 2.4 GHz
+VALU_LANE_OPS = 256 * 4 * 32 * 2.4e9
 CPU_SHARE = 16  # host threads the GPU box allots one GPU's jobs
 
 
@@ -373,7 +375,8 @@ def kernel_rows(q, n=4096, gemm_n=512):
         "us_per_call": round(ms.value * 1e3, 3), "GFLOPs": round(flops / (ms.value * 1e-3) / 1e9, 1),
         "frac_of_valu_floor": round(flops / (ms.value * 1e-3) / VALU_LANE_OPS, 4),
         "note": "the scalar ISA's rounding order (K panels of 256, one serial sum per output per panel): a "
-                "multiply and an add per term on the fp32 VALU, so the floor is 2*M*N*K lane operations"}
+                "multiply (f32 MFMA, which runs on the VALU's units) and an add per term, so the floor is 2*M*N*K "
+                "lane operations"}
     return out
 
 
