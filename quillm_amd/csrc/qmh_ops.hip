@@ -293,8 +293,9 @@ extern "C" int qmh_launch_rope(float *v, int64_t n_heads, int64_t head_dim, cons
 // in that shape, every lane of a load is another cache line, and the address units bound the kernel (131
 // cycles per 1024 products). Four MFMAs go out together: turning the 4 k per lane by lane swaps into
 // k + 4*j + b for one MFMA at a time costs about 20 cycles per swap. Timed, us, 2 x 2 outputs per thread from
-// LDS -> this: 64^3 3.8 -> 3.1, 100x100x1000 26 -> 18, 512^3 15.7 -> 11.2, 1000x1090x1500 129 -> 77, 1024^3 85 -> 52,
-// 2048^3 570 -> 350 (the products and adds alone: 250).
+// LDS -> this, launches in a graph: 64^3 4.1 -> 3.3, 100x100x1000 26 -> 18, 512^3 14.9 -> 10.6, 1000x1090x1500 129 -> 80
+// (91-94 as a single call on an idle card), 1024^3 72 -> 43, 2048^3 530 -> 309 (the products and adds alone: 250), 1x4096x4096
+// 100 -> 65.
 #define QMH_GEMM_KC 256
 #define GN_KG 16  // k per group of four MFMAs
 #define GN_KS 32  // k per chunk (two groups; divides QMH_GEMM_KC)

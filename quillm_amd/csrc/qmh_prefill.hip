@@ -389,12 +389,16 @@ __device__ __forceinline__ void pf_store(const qmh_pf_args &a, int row, int p, f
 // largely add to the VALU's: about 163 cycles per pair of tile and block, and the clock falls to
 // ~1.9 GHz under it. So the shape that needs the fewest cycles wins, not the one with the most work per
 // load: v_mfma_i32_32x32x32_i8 gives 1024 dots in 32 cycles where 16x16x32 takes 64, and likewise the
-// f16 32x32x8 for the scale products. Timed at 512 tokens (us, 16x16 tiles in registers -> this):
-// 12288x4096 150 -> 99, 4096x4096 57 -> 41, W1|W3 2x11008x4096 230 -> 186, 4096x11008 143 -> 95.
+// f16 32x32x8 for the scale products. Timed at 512 tokens (us, 16x16 tiles in registers -> this, launches in a
+// graph over 8 copies of the weights): 12288x4096 125 -> 81, 4096x4096 53 -> 34, W1|W3 2x11008x4096 195 -> 155,
+// 4096x11008 128 -> 81. Counters at W1|W3: 264 cycles per pair of tile and block, 64 of MFMA and 117 of VALU issue;
+// the rest is waves waiting and the last round of workgroups (LDS conflicts 2%).
 // Tried and slower: the int8 accumulator started at the bits of 1.5*2^23 with a second scale product
 // -1.5*2^23*dw*dx, for two VALU instructions per term (an f32 MFMA runs on the VALU's own units, and
 // the third MFMA costs what the conversion saved); 32x32 tiles with operands straight from
-// memory (105, 45, 198, 99: the loads bound it); two token tiles per wave (one wave per SIMD).
+// memory (6 to 10% slower: the loads bound it); two token tiles per wave (one wave per SIMD). Four waves per
+// SIMD are asked of every instance: the 2 x 1 ones hold three (the compiler warns), but asked for three they were 1-2%
+// slower; the Q8_0 2 x 2 ones spill 3-4 registers for the fourth.
 //
 // Operands pass through LDS in stages of PG_KB blocks, two buffers: a thread's pieces of stage i + 2
 // (+ DEEP) are loaded to registers during stage i and written when stage i has been read. The loads'
