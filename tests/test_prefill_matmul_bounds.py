@@ -1,5 +1,6 @@
-"""Index bounds of the tiled prefill matmul's staged loads (k_pf_gemm, quillm_amd/csrc/qmh_prefill.hip),
-modelled on the CPU (no GPU) as tests/test_attn_bounds.py does for the decode attention kernels.
+"""Index bounds of the tiled prefill matmul's staged loads (k_pf_gemm, quillm_amd/csrc/qmh_prefill.hip) and of the f32
+matmul (k_gemm_nt, qmh_ops.hip), modelled on the CPU (no GPU) as tests/test_attn_bounds.py does for the decode
+attention kernels.
 
 The blocks pass in stages of four, and stages are loaded ahead of the one multiplied, so the last loads
 are of blocks past the row's end. Their addresses are a lane offset plus a block offset that a buffer's range
@@ -110,3 +111,33 @@ def test_model_catches_blocks_past_the_end(P, il):
     """Not vacuous: without the last block in their place, the stages past the end leave the arrays."""
     with pytest.raises(AssertionError):
         gemm_loads(4096, 9, 64 if il else 16, il, P, 512, 16, last_block_again=False)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 1, 3), (15, 17, 31), (16, 16, 32), (33, 31, 33), (17, 65, 257), (100, 7, 96)])
+def test_f32_matmul_in_bounds(M, N, K):
+    """k_gemm_nt over grid (ceil(N/32), ceil(M/32)) x 4 waves: the loads of every chunk of 32 k (whole ones as
+    float4s, the last by element), the wave's LDS, the stores; every output once."""
+    KS, LD = 32, 36
+    l = np.arange(64)
+    lr, lk = l >> 3, 4 * (l & 7)
+    nc, nf = (K + KS - 1) // KS, K // KS
+    seen = np.zeros((M, N), int)
+    for wave in range(4):
+        for i0 in range(16 * (wave >> 1), M, 32):
+            for j0 in range(16 * (wave & 1), N, 32):
+                for h in range(2):
+                    for rows, r0 in ((M, i0), (N, j0)):
+                        row = np.minimum(r0 + lr + 8 * h, rows - 1)
+                        for c in range(nc):
+                            for k in range(4):
+                                at = c * KS + lk + k
+                                on = at >= 0 if c < nf else at < K
+                                inb("operand", (row * K + at)[on], rows * K)
+                    inb("LDS write", (lr + 8 * h) * LD + lk + 3, 16 * LD)
+                for g in range(2):
+                    inb("LDS read", (l & 15) * LD + 16 * g + 4 * (l >> 4) + 3, 16 * LD)
+                for e in range(4):
+                    i, j = i0 + 4 * (l >> 4) + e, j0 + (l & 15)
+                    on = (i < M) & (j < N)
+                    np.add.at(seen, (i[on], j[on]), 1)
+    assert (seen == 1).all()
