@@ -405,10 +405,11 @@ __device__ __forceinline__ void pf_store(const qmh_pf_args &a, int row, int p, f
 // offsets are fixed per thread (buffer loads, the block in the scalar offset, which a buffer's range check
 // need not cover). The stages run past the last block, in a last stage that is not whole and in those
 // loaded ahead: these load the last block again, so that every address lies in the matrix, and what they
-// hold is never multiplied. The barrier waits for LDS only, so loads stay in flight across it. Q4_0 codes are written as 16*(q - 8) (two operations per four codes; a chain of 16 x the
-// terms is 16 x the reference's chain exactly, so one multiply by 1/16 ends it: no term is below
-// 2^-48 or above 2^52). In LDS each half block of every row (or token) is contiguous over the rows,
-// which has no bank conflicts; the four fp16 scales of a row sit side by side, and the scale product of
+// hold is never multiplied. The barrier waits for LDS only, so loads stay in flight across it. Q4_0 codes
+// are written as 16*(q - 8) (two operations per four codes; a chain of 16 x the terms is 16 x the
+// reference's chain exactly, so one multiply by 1/16 ends it: no term is below 2^-48 or above 2^52). In LDS
+// each half block of every row (or token) is contiguous over the rows, with 1-2% of the cycles lost to bank
+// conflicts; the four fp16 scales of a row sit side by side, and the scale product of
 // block j takes all four as k = 0..3 of A against B with only entry j (others 0).
 //
 // Inside a block: convert and multiply by the scale products, issue the next block's integer MFMA
